@@ -20,6 +20,7 @@
 namespace orcwa {
 
 typedef double v4d __attribute__((ext_vector_type(4)));
+typedef double v2d __attribute__((ext_vector_type(2)));
 
 static constexpr double kUlp = DBL_EPSILON;
 static constexpr double kSafmin = DBL_MIN;
@@ -500,6 +501,74 @@ __device__ inline bool small_subdiag(const cd* H, int n, int k, int lo, int hi, 
     if (ba * (ab / s) <= fmax(smlnum, kUlp * (bb * (aa / s)))) return true;
   }
   return false;
+}
+
+// ---------------------------------------------------------------------------
+// 2x2 unitary rotations with a real c: G = [[c, -conj(s)], [s, c]],
+// G^H (x0, x1) = (r, 0).  A row or column pair then takes 12 real operations
+// (16 with c complex), which is what bounds the QR's chase in LDS.
+// ---------------------------------------------------------------------------
+struct Rot {
+  double c;
+  cd s, r;
+};
+
+// 1 / sqrt(v) to 2 ulp: the hardware's estimate (about 24 bits) and two Newton
+// steps.  A third of the latency of a square root and a division, on the chain
+// that every rotation waits for.
+__device__ __forceinline__ double rsqrt_n(double v) {
+  const double h = -0.5 * v;
+  double y = __builtin_amdgcn_rsq(v);
+  y = fma(y, fma(h * y, y, 0.5), y);
+  return fma(y, fma(h * y, y, 0.5), y);
+}
+// root and reciprocal to about 44 bits, for shifts
+__device__ __forceinline__ double sqrt_shift(double v) {
+  if (!(v > 1e-280)) return 0.0;
+  double y = __builtin_amdgcn_rsq(v);
+  y = fma(y, fma(-0.5 * v * y, y, 0.5), y);
+  return v * y;
+}
+__device__ __forceinline__ double rcp_shift(double v) {
+  const double y = __builtin_amdgcn_rcp(v);
+  return fma(y, fma(-v, y, 1.0), y);
+}
+
+// the rotation, where neither norm is near the ends of the range (false otherwise)
+__device__ __forceinline__ bool rot_gen_fast(cd x0, cd x1, Rot& g) {
+  const double n0 = norm2(x0), n = n0 + norm2(x1);
+  const double t = rsqrt_n(n0) * rsqrt_n(n);
+  g.c = n0 * t;
+  g.s = t * mulc(x1, x0);
+  g.r = (n * t) * x0;
+  return n0 > 1e-280 && n < 1e280;
+}
+__device__ __forceinline__ Rot rot_gen(cd x0, cd x1) {
+  Rot g;
+  if (rot_gen_fast(x0, x1, g)) return g;
+  const double m0 = fmax(fabs(x0.re), fabs(x0.im)), m1 = fmax(fabs(x1.re), fabs(x1.im));
+  if (m1 == 0.0) {
+    g.c = 1.0;
+    g.s = mk(0.0, 0.0);
+    g.r = x0;
+    return g;
+  }
+  const double m = fmax(m0, m1), im = 1.0 / m;
+  const cd y1 = im * x1;
+  if (m0 < 1e-150 * m1) {      // x0 does not count
+    const double a1 = sqrt(norm2(y1));
+    g.c = 0.0;
+    g.s = (1.0 / a1) * y1;
+    g.r = mk(m * a1, 0.0);
+    return g;
+  }
+  const cd y0 = im * x0;
+  const double a0 = hypot(y0.re, y0.im), a = sqrt(norm2(y0) + norm2(y1));
+  const cd u0 = (1.0 / a0) * y0;   // phase of x0
+  g.c = a0 / a;
+  g.s = (1.0 / a) * mulc(y1, u0);
+  g.r = (m * a) * u0;
+  return g;
 }
 
 // ---------------------------------------------------------------------------
