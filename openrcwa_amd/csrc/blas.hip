@@ -92,9 +92,9 @@ __global__ __launch_bounds__(256, 2) void k_zgemm(
 
   int bx, by, b;
   tile_of_block(bx, by, b);
-  const cd* __restrict__ A = Ap[b] + offA;
-  const cd* __restrict__ B = Bp[b] + offB;
-  cd* __restrict__ C = Cp[b] + offC;
+  const cd* __restrict__ A = gptr(Ap[b]) + offA;
+  const cd* __restrict__ B = gptr(Bp[b]) + offB;
+  cd* __restrict__ C = gptr(Cp[b]) + offC;
   const int m0 = bx * TM, n0 = by * TN;
   // op(B) upper triangular from diagonal kup on: its rows past this tile's
   // last column + kup are zero, so the K range ends there
@@ -106,8 +106,7 @@ __global__ __launch_bounds__(256, 2) void k_zgemm(
   // global loads run along whichever index of an operand has unit stride
   const bool a_mfast = (rsA == 1), b_kfast = (rsB == 1);
   int amm[LA], akk[LA], bkk[LB], bnn[LB];
-  const cd* pa[LA];
-  const cd* pb[LB];
+  long long pa[LA], pb[LB];
   bool aok[LA], bok[LB];
 #pragma unroll
   for (int j = 0; j < LA; ++j) {
@@ -115,7 +114,7 @@ __global__ __launch_bounds__(256, 2) void k_zgemm(
     amm[j] = a_mfast ? (e % TM) : (e / GEMM_KS);
     akk[j] = a_mfast ? (e / TM) : (e % GEMM_KS);
     aok[j] = (m0 + amm[j] < M);
-    pa[j] = A + (long long)(m0 + amm[j]) * rsA + (long long)akk[j] * csA;
+    pa[j] = (long long)(m0 + amm[j]) * rsA + (long long)akk[j] * csA;
   }
 #pragma unroll
   for (int j = 0; j < LB; ++j) {
@@ -123,14 +122,14 @@ __global__ __launch_bounds__(256, 2) void k_zgemm(
     bkk[j] = b_kfast ? (e % GEMM_KS) : (e / TN);
     bnn[j] = b_kfast ? (e / GEMM_KS) : (e % TN);
     bok[j] = (n0 + bnn[j] < N);
-    pb[j] = B + (long long)bkk[j] * rsB + (long long)(n0 + bnn[j]) * csB;
+    pb[j] = (long long)bkk[j] * rsB + (long long)(n0 + bnn[j]) * csB;
   }
   const long long stepA = GEMM_KS * csA, stepB = GEMM_KS * rsB;
   cd ra[LA], rb[LB];
 #pragma unroll
-  for (int j = 0; j < LA; ++j) ra[j] = (aok[j] && akk[j] < K) ? pa[j][0] : mk(0.0, 0.0);
+  for (int j = 0; j < LA; ++j) ra[j] = (aok[j] && akk[j] < K) ? A[pa[j]] : mk(0.0, 0.0);
 #pragma unroll
-  for (int j = 0; j < LB; ++j) rb[j] = (bok[j] && bkk[j] < K) ? pb[j][0] : mk(0.0, 0.0);
+  for (int j = 0; j < LB; ++j) rb[j] = (bok[j] && bkk[j] < K) ? B[pb[j]] : mk(0.0, 0.0);
 
   // Gauss form: T1 = ar br, T2 = ai bi, T3 = (ar + ai)(br + bi);
   // re = T1 - T2, im = T3 - T1 - T2 (three real MFMAs per complex product)
@@ -161,12 +160,12 @@ __global__ __launch_bounds__(256, 2) void k_zgemm(
 #pragma unroll
       for (int j = 0; j < LA; ++j) {
         pa[j] += stepA;
-        ra[j] = (aok[j] && k0 + GEMM_KS + akk[j] < K) ? pa[j][0] : mk(0.0, 0.0);
+        ra[j] = (aok[j] && k0 + GEMM_KS + akk[j] < K) ? A[pa[j]] : mk(0.0, 0.0);
       }
 #pragma unroll
       for (int j = 0; j < LB; ++j) {
         pb[j] += stepB;
-        rb[j] = (bok[j] && k0 + GEMM_KS + bkk[j] < K) ? pb[j][0] : mk(0.0, 0.0);
+        rb[j] = (bok[j] && k0 + GEMM_KS + bkk[j] < K) ? B[pb[j]] : mk(0.0, 0.0);
       }
     }
 #pragma unroll
@@ -255,9 +254,9 @@ __global__ __launch_bounds__(256, 2) void k_zgemm_f32(
   __shared__ float sBr[KS][TN + 1], sBi[KS][TN + 1];
   int bx, by, b;
   tile_of_block(bx, by, b);
-  const cd* __restrict__ A = Ap[b] + offA;
-  const cd* __restrict__ B = Bp[b] + offB;
-  cd* __restrict__ C = Cp[b] + offC;
+  const cd* __restrict__ A = gptr(Ap[b]) + offA;
+  const cd* __restrict__ B = gptr(Bp[b]) + offB;
+  cd* __restrict__ C = gptr(Cp[b]) + offC;
   const int m0 = bx * TM, n0 = by * TN;
   // op(B) upper triangular from diagonal kup on: its rows past this tile's
   // last column + kup are zero, so the K range ends there
@@ -267,8 +266,7 @@ __global__ __launch_bounds__(256, 2) void k_zgemm_f32(
   const double sa = conjA ? -1.0 : 1.0, sb = conjB ? -1.0 : 1.0;
   const bool a_mfast = (rsA == 1), b_kfast = (rsB == 1);
   int amm[LA], akk[LA], bkk[LB], bnn[LB];
-  const cd* pa[LA];
-  const cd* pb[LB];
+  long long pa[LA], pb[LB];
   bool aok[LA], bok[LB];
 #pragma unroll
   for (int j = 0; j < LA; ++j) {
@@ -276,7 +274,7 @@ __global__ __launch_bounds__(256, 2) void k_zgemm_f32(
     amm[j] = a_mfast ? (e % TM) : (e / KS);
     akk[j] = a_mfast ? (e / TM) : (e % KS);
     aok[j] = (m0 + amm[j] < M);
-    pa[j] = A + (long long)(m0 + amm[j]) * rsA + (long long)akk[j] * csA;
+    pa[j] = (long long)(m0 + amm[j]) * rsA + (long long)akk[j] * csA;
   }
 #pragma unroll
   for (int j = 0; j < LB; ++j) {
@@ -284,14 +282,14 @@ __global__ __launch_bounds__(256, 2) void k_zgemm_f32(
     bkk[j] = b_kfast ? (e % KS) : (e / TN);
     bnn[j] = b_kfast ? (e / KS) : (e % TN);
     bok[j] = (n0 + bnn[j] < N);
-    pb[j] = B + (long long)bkk[j] * rsB + (long long)(n0 + bnn[j]) * csB;
+    pb[j] = (long long)bkk[j] * rsB + (long long)(n0 + bnn[j]) * csB;
   }
   const long long stepA = KS * csA, stepB = KS * rsB;
   cd ra[LA], rb[LB];
 #pragma unroll
-  for (int j = 0; j < LA; ++j) ra[j] = (aok[j] && akk[j] < K) ? pa[j][0] : mk(0.0, 0.0);
+  for (int j = 0; j < LA; ++j) ra[j] = (aok[j] && akk[j] < K) ? A[pa[j]] : mk(0.0, 0.0);
 #pragma unroll
-  for (int j = 0; j < LB; ++j) rb[j] = (bok[j] && bkk[j] < K) ? pb[j][0] : mk(0.0, 0.0);
+  for (int j = 0; j < LB; ++j) rb[j] = (bok[j] && bkk[j] < K) ? B[pb[j]] : mk(0.0, 0.0);
 
   double d1[BI][BJ][4], d2[BI][BJ][4], d3[BI][BJ][4];
 #pragma unroll
@@ -317,12 +315,12 @@ __global__ __launch_bounds__(256, 2) void k_zgemm_f32(
 #pragma unroll
       for (int j = 0; j < LA; ++j) {
         pa[j] += stepA;
-        ra[j] = (aok[j] && k0 + KS + akk[j] < K) ? pa[j][0] : mk(0.0, 0.0);
+        ra[j] = (aok[j] && k0 + KS + akk[j] < K) ? A[pa[j]] : mk(0.0, 0.0);
       }
 #pragma unroll
       for (int j = 0; j < LB; ++j) {
         pb[j] += stepB;
-        rb[j] = (bok[j] && k0 + KS + bkk[j] < K) ? pb[j][0] : mk(0.0, 0.0);
+        rb[j] = (bok[j] && k0 + KS + bkk[j] < K) ? B[pb[j]] : mk(0.0, 0.0);
       }
     }
     v4f p1[BI][BJ], p2[BI][BJ], p3[BI][BJ];
@@ -421,9 +419,9 @@ __global__ __launch_bounds__(256, 2) void k_zgemm_bf16(
   __shared__ __attribute__((aligned(16))) __bf16 sB[2][S][TN][LDK];
   int bx, by, b;
   tile_of_block(bx, by, b);
-  const cd* __restrict__ A = Ap[b] + offA;
-  const cd* __restrict__ B = Bp[b] + offB;
-  cd* __restrict__ C = Cp[b] + offC;
+  const cd* __restrict__ A = gptr(Ap[b]) + offA;
+  const cd* __restrict__ B = gptr(Bp[b]) + offB;
+  cd* __restrict__ C = gptr(Cp[b]) + offC;
   const int m0 = bx * TM, n0 = by * TN;
   // op(B) upper triangular from diagonal kup on: its rows past this tile's
   // last column + kup are zero, so the K range ends there
@@ -674,7 +672,7 @@ __global__ __launch_bounds__(256) void k_getf2_panel(int n, int k0, int nb, cd* 
   __shared__ int s_piv;
   __shared__ cd s_u[NB];
   const int b = blockIdx.x;
-  cd* __restrict__ A = Ap[b];
+  cd* __restrict__ A = gptr(Ap[b]);
   const int tid = threadIdx.x;
   for (int j = 0; j < nb; ++j) {
     const int c = k0 + j;
@@ -844,7 +842,7 @@ __global__ __launch_bounds__(GF_T) void k_getf2_reg(int n, int k0, int nb, cd* c
   S.ipiv = ipiv;
   S.info = info;
   S.info_map = info_map;
-  cd* __restrict__ A = Ap[S.b];
+  cd* __restrict__ A = gptr(Ap[S.b]);
   cd a[NB];
 #pragma unroll
   for (int j = 0; j < NB; ++j)
@@ -862,7 +860,7 @@ __global__ void k_laswp(int n, int ncols_total, int k0, int nb, int c0, int c1, 
   const int b = blockIdx.y;
   const int col = c0 + blockIdx.x * blockDim.x + threadIdx.x;
   if (col >= c1 || col >= ncols_total) return;
-  cd* __restrict__ A = Ap[b] + (long long)col * n;
+  cd* __restrict__ A = gptr(Ap[b]) + (long long)col * n;
   const int* pv = ipiv + (long long)b * n;
   for (int j = 0; j < nb; ++j) {
     const int r = k0 + j;
@@ -911,7 +909,7 @@ __global__ __launch_bounds__(256) void k_laswp_panel(int n, int k0, int nb, int 
   const int ns = s_ns;
   const int c = threadIdx.x % LASWP_NC, sg = threadIdx.x / LASWP_NC;
   const int col = c0 + blockIdx.x * LASWP_NC + c;
-  cd* __restrict__ A = Ap[b] + (long long)col * n;
+  cd* __restrict__ A = gptr(Ap[b]) + (long long)col * n;
   if (col < c1)
     for (int t = sg; t < ns; t += 256 / LASWP_NC) tile[t][c] = A[R[t]];
   __syncthreads();
@@ -951,7 +949,7 @@ __global__ __launch_bounds__(256) void k_apply_perm(int n, int nrhs, int ncw, co
   extern __shared__ cd X[];   // [ncw][n]
   const int b = blockIdx.y;
   const int c0 = blockIdx.x * ncw;
-  cd* __restrict__ B = Bp[b];
+  cd* __restrict__ B = gptr(Bp[b]);
   const int* pm = perm + (long long)b * n;
   const int nc = min(ncw, nrhs - c0);
   for (int e = threadIdx.x; e < nc * n; e += 256) {
@@ -979,8 +977,8 @@ __global__ __launch_bounds__(256) void k_trsm_block(int n, int k0, int nb, int c
   __shared__ cd sT[NB][NB];
   __shared__ cd sX[256][TR_SLAB + 1];
   const int b = blockIdx.y;
-  const cd* __restrict__ Lm = Lp[b];
-  cd* __restrict__ X = Xp[b];
+  const cd* __restrict__ Lm = gptr(Lp[b]);
+  cd* __restrict__ X = gptr(Xp[b]);
   const int tid = threadIdx.x;
   // (zero outside nb x nb, so the unrolled products below need no guard)
   for (int e = tid; e < NB * NB; e += 256) {
@@ -1135,7 +1133,7 @@ void zgetrs_batched(hipStream_t s, int n, int nrhs, const cd* const* LU, const i
 // elementwise
 // ---------------------------------------------------------------------------
 __global__ void k_set_identity(int n, cd* const* Ap) {
-  cd* A = Ap[blockIdx.y];
+  cd* A = gptr(Ap[blockIdx.y]);
   const long long nn = (long long)n * n;
   for (long long e = blockIdx.x * (long long)blockDim.x + threadIdx.x; e < nn;
        e += (long long)gridDim.x * blockDim.x) {
@@ -1146,17 +1144,17 @@ __global__ void k_set_identity(int n, cd* const* Ap) {
 
 __global__ void k_axpby(long long count, cd a, const cd* const* Ap, cd bb, const cd* const* Bp,
                         cd* const* Cp) {
-  const cd* A = Ap[blockIdx.y];
-  const cd* B = Bp[blockIdx.y];
-  cd* C = Cp[blockIdx.y];
+  const cd* A = gptr(Ap[blockIdx.y]);
+  const cd* B = gptr(Bp[blockIdx.y]);
+  cd* C = gptr(Cp[blockIdx.y]);
   for (long long e = blockIdx.x * (long long)blockDim.x + threadIdx.x; e < count;
        e += (long long)gridDim.x * blockDim.x)
     C[e] = a * A[e] + bb * B[e];
 }
 
 __global__ void k_copy(long long count, const cd* const* Ap, cd* const* Bp) {
-  const cd* A = Ap[blockIdx.y];
-  cd* B = Bp[blockIdx.y];
+  const cd* A = gptr(Ap[blockIdx.y]);
+  cd* B = gptr(Bp[blockIdx.y]);
   for (long long e = blockIdx.x * (long long)blockDim.x + threadIdx.x; e < count;
        e += (long long)gridDim.x * blockDim.x)
     B[e] = A[e];

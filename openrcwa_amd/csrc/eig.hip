@@ -50,7 +50,7 @@ __global__ __launch_bounds__(256) void k_hess(int n, cd* const* Ap, cd* tau_all)
   __shared__ cd s_tau, s_scale;
 
   const int b = blockIdx.x;
-  cd* __restrict__ A = Ap[b];
+  cd* __restrict__ A = gptr(Ap[b]);
   cd* tau = tau_all + (long long)b * n;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
 
@@ -174,8 +174,8 @@ __global__ __launch_bounds__(256) void k_hess_panel(int n, int i0, int nb, cd* c
   __shared__ cd s_tau, s_scale;
 
   const int mat = blockIdx.x;
-  cd* __restrict__ A = Ap[mat];
-  cd* __restrict__ V = Xp[mat];
+  cd* __restrict__ A = gptr(Ap[mat]);
+  cd* __restrict__ V = gptr(Xp[mat]);
   cd* __restrict__ Y = V + (long long)n * HB;
   cd* __restrict__ Tg = V + 3LL * n * HB;
   cd* tau = tau_all + (long long)mat * n;
@@ -363,8 +363,8 @@ __global__ __launch_bounds__(256) void k_formq(int n, const cd* const* Ap, const
   cd* sv = sm;
   cd* sw = sm + n;
   const int b = blockIdx.x;
-  const cd* __restrict__ A = Ap[b];
-  cd* __restrict__ Z = Zp[b];
+  const cd* __restrict__ A = gptr(Ap[b]);
+  cd* __restrict__ Z = gptr(Zp[b]);
   const cd* tau = tau_all + (long long)b * n;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const long long nn = (long long)n * n;
@@ -409,8 +409,8 @@ constexpr int QB = 32;
 
 // Vall[:, j] = reflector j as a dense column (zeros above row j+1, 1 at j+1)
 __global__ void k_extract_v(int n, const cd* const* Ap, cd* const* Vp) {
-  const cd* A = Ap[blockIdx.y];
-  cd* V = Vp[blockIdx.y];
+  const cd* A = gptr(Ap[blockIdx.y]);
+  cd* V = gptr(Vp[blockIdx.y]);
   const long long cnt = (long long)n * (n - 2);
   for (long long e = blockIdx.x * (long long)blockDim.x + threadIdx.x; e < cnt;
        e += (long long)gridDim.x * blockDim.x) {
@@ -433,7 +433,7 @@ __global__ __launch_bounds__(256) void k_larft(int n, const cd* const* Vp, const
   const int nref = n - 2;
   const int j0 = blk * QB;
   const int nbk = min(QB, nref - j0);
-  const cd* V = Vp[b];
+  const cd* V = gptr(Vp[b]);
   const cd* tau = tau_all + (long long)b * n;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   // G = V_b^H V_b (upper part needed), rows from j0+1 (above: zeros)
@@ -469,7 +469,7 @@ __global__ __launch_bounds__(256) void k_larft(int n, const cd* const* Vp, const
     }
   }
   __syncthreads();
-  cd* T = Tp[b] + (long long)blk * QB * QB;
+  cd* T = gptr(Tp[b]) + (long long)blk * QB * QB;
   for (int e = tid; e < QB * QB; e += 256) {
     const int r = e % QB, c = e / QB;
     T[e] = (r < nbk && c < nbk) ? Tl[r][c] : mk(0.0, 0.0);
@@ -610,8 +610,8 @@ namespace qr_w64 {
 // ---------------------------------------------------------------------------
 __global__ __launch_bounds__(256) void k_trevc(int n, const cd* const* Tp, cd* const* Xp) {
   const int b = blockIdx.x;
-  const cd* __restrict__ T = Tp[b];
-  cd* __restrict__ X = Xp[b];
+  const cd* __restrict__ T = gptr(Tp[b]);
+  cd* __restrict__ X = gptr(Xp[b]);
   const int tid = threadIdx.x;
   const long long nn = (long long)n * n;
   const double smlnum = kSafmin * ((double)n / kUlp);
@@ -655,8 +655,8 @@ __global__ __launch_bounds__(256) void k_trevc_block(int n, int i0, int i1, cons
                                                      cd* const* Xp) {
   __shared__ cd Tb[TB][TB + 1];
   const int b = blockIdx.y;
-  const cd* __restrict__ T = Tp[b];
-  cd* __restrict__ X = Xp[b];
+  const cd* __restrict__ T = gptr(Tp[b]);
+  cd* __restrict__ X = gptr(Xp[b]);
   const int nb = i1 - i0;
   for (int e = threadIdx.x; e < TB * TB; e += 256) {
     const int r = e % TB, c = e / TB;
@@ -710,8 +710,8 @@ static void trevc_blocked(hipStream_t s, int n, const cd* const* T, cd* const* X
 __global__ __launch_bounds__(256) void k_eig_finish(int n, const cd* const* Tp, cd* const* Wp,
                                                     cd* lam) {
   const int b = blockIdx.x;
-  const cd* T = Tp[b];
-  cd* W = Wp[b];
+  const cd* T = gptr(Tp[b]);
+  cd* W = gptr(Wp[b]);
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   for (int j = tid; j < n; j += 256) lam[(long long)b * n + j] = T[j + (long long)j * n];
   for (int j = wave; j < n; j += 4) {
@@ -732,9 +732,9 @@ __global__ __launch_bounds__(256) void k_eig_residual(int n, const cd* const* Ap
                                                       double tol) {
   __shared__ double sred[4];
   const int b = blockIdx.x;
-  const cd* A = Ap[b];
-  const cd* W = Wp[b];
-  const cd* R = Rp[b];
+  const cd* A = gptr(Ap[b]);
+  const cd* W = gptr(Wp[b]);
+  const cd* R = gptr(Rp[b]);
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const long long nn = (long long)n * n;
   double ma = 0.0, mr = 0.0;
@@ -761,7 +761,7 @@ __global__ __launch_bounds__(256) void k_eig_residual(int n, const cd* const* Ap
 }
 
 __global__ void k_zero_below_subdiag(int n, cd* const* Ap) {
-  cd* Am = Ap[blockIdx.y];
+  cd* Am = gptr(Ap[blockIdx.y]);
   const long long nn = (long long)n * n;
   for (long long e = blockIdx.x * (long long)blockDim.x + threadIdx.x; e < nn;
        e += (long long)gridDim.x * blockDim.x) {
@@ -777,8 +777,8 @@ __global__ void k_zero_below_subdiag(int n, cd* const* Ap) {
 __global__ __launch_bounds__(256) void k_perturb_diag(int n, const cd* const* Aop,
                                                       cd* const* Ap) {
   __shared__ double sm[4];
-  const cd* Ao = Aop[blockIdx.x];
-  cd* A = Ap[blockIdx.x];
+  const cd* Ao = gptr(Aop[blockIdx.x]);
+  cd* A = gptr(Ap[blockIdx.x]);
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const long long nn = (long long)n * n;
   double m = 0.0;

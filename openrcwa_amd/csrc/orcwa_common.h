@@ -73,6 +73,15 @@ __host__ __device__ inline cd cexp(cd z) {
   return mk(e * c, e * s);
 }
 
+// A pointer read from a device table has no known address space, so the compiler
+// moves everything behind it with flat instructions: those also count as LDS
+// accesses, and waiting for an LDS read then waits for every load in flight.
+// Rebuilt from its integer value in the global address space, it is known.
+template <class T>
+__device__ __forceinline__ T* gptr(T* p) {
+  return (T*)((__attribute__((address_space(1))) T*)(unsigned long long)p);
+}
+
 // wavefront (64-lane) helpers
 __device__ inline double wave_sum(double v) {
   for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);

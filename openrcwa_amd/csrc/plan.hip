@@ -1110,8 +1110,8 @@ static int eig_recover(orcwa_plan* p, const ChunkTables& ct, hipStream_t s,
 }
 
 __global__ void k_scale_rows_keff(int n, cd* const* Hp, const cd* const* Kp) {
-  cd* H = Hp[blockIdx.y];
-  const cd* kf = Kp[blockIdx.y];
+  cd* H = gptr(Hp[blockIdx.y]);
+  const cd* kf = gptr(Kp[blockIdx.y]);
   const long long count = (long long)n * n;
   for (long long e = blockIdx.x * (long long)blockDim.x + threadIdx.x; e < count;
        e += (long long)gridDim.x * blockDim.x)

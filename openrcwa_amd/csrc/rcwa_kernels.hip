@@ -249,8 +249,8 @@ __global__ void k_build_pq(const ConvGeom g, const ProbParam* params, const Grid
     v12.re += kxr * kyr;
     v22.re -= kxr * kxr;
   }
-  cd* P = PQ[pi];
-  cd* P2 = PQcopy[pi];
+  cd* P = gptr(PQ[pi]);
+  cd* P2 = gptr(PQcopy[pi]);
   const long long i11 = r + (long long)c * n, i21 = (h + r) + (long long)c * n;
   const long long i12 = r + (long long)(h + c) * n, i22 = (h + r) + (long long)(h + c) * n;
   P[i11] = v11; P[i21] = v21; P[i12] = v12; P[i22] = v22;
@@ -279,8 +279,8 @@ __global__ void k_build_v(const ConvGeom g, const ProbParam* params, const cd* c
   const int rr = (r < h) ? r : r - h;
   double kx, ky;
   k_vectors(g, p, rr, kx, ky);
-  const cd* w = W[pi] + (long long)c * n;
-  const cd* q = QW1[pi] + (long long)c * n;
+  const cd* w = gptr(W[pi]) + (long long)c * n;
+  const cd* q = gptr(QW1[pi]) + (long long)c * n;
   cd v;
   if (r < h) v = (-(kx * ky)) * w[rr] + (kx * kx) * w[h + rr] - q[rr];
   else v = q[h + rr] - (ky * ky) * w[rr] + (ky * kx) * w[h + rr];
@@ -306,8 +306,8 @@ __global__ void k_build_pq_mag(const ConvGeom g, const ProbParam* params, const 
   k_vectors(g, p, r, kxr, kyr);
   k_vectors(g, p, c, kxc, kyc);
   const cd ei = M.Ei[e], mi = M.Mi[e];
-  cd* P = Pp[pi];
-  cd* Q = Qp[pi];
+  cd* P = gptr(Pp[pi]);
+  cd* Q = gptr(Qp[pi]);
   const long long i11 = r + (long long)c * n, i21 = (h + r) + (long long)c * n;
   const long long i12 = r + (long long)(h + c) * n, i22 = (h + r) + (long long)(h + c) * n;
   P[i11] = (kxr * kyc) * ei;
@@ -339,7 +339,7 @@ __global__ void k_build_v_mag(int n, const cd* const* QW, const cd* lam, cd* kef
 }
 
 __global__ void k_zero_mats(long long count, cd* const* A) {
-  cd* a = A[blockIdx.y];
+  cd* a = gptr(A[blockIdx.y]);
   for (long long e = blockIdx.x * (long long)blockDim.x + threadIdx.x; e < count;
        e += (long long)gridDim.x * blockDim.x)
     a[e] = mk(0.0, 0.0);
@@ -357,7 +357,7 @@ __global__ void k_uniform(const ConvGeom g, const UniParam* params, cd* keff_all
   const UniParam u = params[ui];
   const int h = g.nx * g.ny, n = 2 * h;
   const long long nn = (long long)n * n;
-  cd* V = Vdense[ui];
+  cd* V = gptr(Vdense[ui]);
   (void)nn;
   const int k = blockIdx.x * blockDim.x + threadIdx.x;
   if (k >= h) return;
@@ -405,10 +405,10 @@ __global__ void k_bdinv_apply(int h, const cd* const* binv, const cd* const* Vb,
   const long long e = blockIdx.x * (long long)blockDim.x + threadIdx.x;
   if (e >= cnt) return;
   const int k = (int)(e % h), c = (int)(e / h);
-  const cd* bi = binv[b];
-  const cd* v = Vb[b] + (long long)c * n;
+  const cd* bi = gptr(binv[b]);
+  const cd* v = gptr(Vb[b]) + (long long)c * n;
   const cd x0 = v[k], x1 = v[h + k];
-  cd* o = Hout[b] + (long long)c * n;
+  cd* o = gptr(Hout[b]) + (long long)c * n;
   o[k] = bi[k] * x0 + bi[h + k] * x1;
   o[h + k] = bi[2 * h + k] * x0 + bi[3 * h + k] * x1;
 }
@@ -425,7 +425,7 @@ __global__ void k_phase_scale(int n, const cd* const* keff, const double* k0d, c
   const int b = blockIdx.y;
   const long long nn = (long long)n * n;
   const double kd = k0d[b];
-  const cd* kf = keff[b];
+  const cd* kf = gptr(keff[b]);
   for (long long e = blockIdx.x * (long long)blockDim.x + threadIdx.x; e < nn;
        e += (long long)gridDim.x * blockDim.x) {
     const int r = (int)(e % n), c = (int)(e / n);
@@ -459,11 +459,11 @@ __global__ void k_sum_diff_t(int n, cd* const* Ep, cd* const* Hp, const cd* cons
                              cd* const* Atp, cd* const* Btp) {
   __shared__ cd ta[32][33], tb[32][33];
   const int z = blockIdx.z;
-  cd* E = Ep[z];
-  cd* H = Hp[z];
-  const cd* kf = keff_a[z];
-  cd* At = Atp[z];
-  cd* Bt = Btp ? Btp[z] : nullptr;
+  cd* E = gptr(Ep[z]);
+  cd* H = gptr(Hp[z]);
+  const cd* kf = gptr(keff_a[z]);
+  cd* At = gptr(Atp[z]);
+  cd* Bt = Btp ? gptr(Btp[z]) : nullptr;
   const int r0 = blockIdx.x * 32, c0 = blockIdx.y * 32;
   const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;   // 256 threads: 32 x 8
   for (int k = ty; k < 32; k += 8) {
@@ -501,8 +501,8 @@ __global__ void k_pv_in(const ConvGeom g, const ProbParam* params, const cd* con
   const int b = blockIdx.y;
   const ProbParam p = params[b];
   const int h = g.nx * g.ny, n = 2 * h;
-  const cd* V = Vb[b];
-  cd* O = out[b];
+  const cd* V = gptr(Vb[b]);
+  cd* O = gptr(out[b]);
   const long long cnt = (long long)h * n;
   for (long long e = blockIdx.x * (long long)blockDim.x + threadIdx.x; e < cnt;
        e += (long long)gridDim.x * blockDim.x) {
@@ -519,9 +519,9 @@ __global__ void k_pv_out(const ConvGeom g, const ProbParam* params, const cd* co
   const int b = blockIdx.y;
   const ProbParam p = params[b];
   const int h = g.nx * g.ny, n = 2 * h;
-  const cd* U = Up[b] + offU;
-  const cd* V = Vb[b];
-  cd* H = Hp[b];
+  const cd* U = gptr(Up[b]) + offU;
+  const cd* V = gptr(Vb[b]);
+  cd* H = gptr(Hp[b]);
   const long long cnt = (long long)n * n;
   for (long long e = blockIdx.x * (long long)blockDim.x + threadIdx.x; e < cnt;
        e += (long long)gridDim.x * blockDim.x) {
@@ -547,6 +547,7 @@ constexpr int TS = 32;
 __device__ void lu_t_solve2(int n, const cd* __restrict__ LU,
                             const int* __restrict__ piv, cd* x0, cd* x1,
                             cd (*blk)[TS + 1]) {
+  LU = gptr(LU);
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int nblk = (n + TS - 1) / TS;
   // U^T y = x, forward: y_i = (x_i - sum_{j<i} U(j,i) y_j) / U(i,i)
@@ -689,7 +690,7 @@ __global__ __launch_bounds__(256) void k_cascade_tail(int n, int i0, const cd* c
   lu_t_solve2(n, LUt[b], piv_all + (long long)b * n, x0, x1,
               reinterpret_cast<cd(*)[TS + 1]>(u0));
   // u = R~ x, R~(i, j) = Rt(j, i): column i of Rt
-  const cd* Rt = Rtp ? Rtp[b] : nullptr;
+  const cd* Rt = Rtp ? gptr(Rtp[b]) : nullptr;
   for (int i = wave; i < n; i += 4) {
     double a0r = 0.0, a0i = 0.0, a1r = 0.0, a1i = 0.0;
     if (Rt) {
@@ -712,8 +713,8 @@ __global__ __launch_bounds__(256) void k_cascade_tail(int n, int i0, const cd* c
     }
   }
   __syncthreads();
-  const cd* A = Ap[b];
-  const cd* B = Bp[b];
+  const cd* A = gptr(Ap[b]);
+  const cd* B = gptr(Bp[b]);
   cd* out = rt_all + (long long)b * 4 * n;
   for (int i = tid; i < n; i += 256) {
     cd r0 = mk(0.0, 0.0), r1 = mk(0.0, 0.0);
@@ -740,7 +741,7 @@ __global__ __launch_bounds__(256) void k_cascade_chain(int n, const cd* const* L
   cd* x1 = sm + n;
   const int b = blockIdx.x, tid = threadIdx.x;
   cd* t = rt_all + (long long)b * 4 * n + 2 * n;
-  const cd* kf = keff[b];
+  const cd* kf = gptr(keff[b]);
   const double kd = k0d[b];
   for (int i = tid; i < n; i += 256) {
     const cd a = kd * kf[i];
