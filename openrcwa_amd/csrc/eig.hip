@@ -571,16 +571,60 @@ __device__ __forceinline__ Rot rot_gen(cd x0, cd x1) {
   return g;
 }
 
+// State of one matrix's iteration and the unitaries of a round (section 3c of
+// qr_ms.inc), at the start of its X slot.
+struct QrOp {
+  int a, wa;      // rows and columns [a, a + wa)
+  int rl, ch;     // not yet applied to rows [0, rl) and columns [ch, n)
+  int off, ld;    // the unitary (ld x ld, zero past wa): X + off, or W + (-1 - off)
+};
+constexpr int QR_MAX_OPS = 288;
+struct QrRound {
+  int hi, sweeps, noprog, nops;
+  QrOp op[QR_MAX_OPS];
+};
+constexpr int QR_BLOCK = 48;       // window of the sweeps
+constexpr int QR_MAX_AED = 6;      // early deflations of a round
+constexpr int QR_AED_NW = 24, QR_AED_BLOCK = 32;   // early-deflation window, its LDS block
+constexpr int QR_HDR = 448;        // (in cd)
+constexpr int QR_SLOT0 = QR_HDR + QR_MAX_AED * QR_AED_BLOCK * QR_AED_BLOCK;
+static_assert(sizeof(QrRound) <= QR_HDR * sizeof(cd), "QR round header");
+// 48 x 48 unitaries that X, and X and W, hold
+__host__ __device__ constexpr int qr_slots_x(int n) {
+  return n * n > QR_SLOT0 ? (n * n - QR_SLOT0) / (QR_BLOCK * QR_BLOCK) : 0;
+}
+__host__ __device__ constexpr int qr_slots(int n) {
+  return qr_slots_x(n) + n * n / (QR_BLOCK * QR_BLOCK);
+}
+// Whether the QR of `batch` matrices runs in rounds (section 3c of qr_ms.inc).
+// The unitaries of a round have to fit X and W (a sweep's windows start 2 QNS - 1
+// rows apart, but for a few at the ends).  A round lasts as long as its slowest
+// matrix, so the more matrices there are, the more is lost against one
+// workgroup a matrix running through; the larger n is, the more the applies
+// gain.  One pillar stack of 4 layers, ms in rounds / in one kernel: n = 242
+// with 4 matrices 57.8 / 58.1, 32: 66 / 60; n = 338, 4: 91 / 100, 40: 114 / 109;
+// n = 450, 4: 136 / 158, 20: 168 / 177, 80: 205 / 203, 256: 294 / 261; n = 722,
+// 3: 321 / 426, 60: 484 / 544: about even at batch = n^2 / 8000.
+__host__ constexpr bool qr_split(int n, int batch) {
+  const int need = (n - QR_BLOCK) / 10 + 4;
+  return n >= 128 && qr_slots(n) >= need && need + QR_MAX_AED <= QR_MAX_OPS &&
+         8000LL * batch <= (long long)n * n;
+}
+
 // ---------------------------------------------------------------------------
 // 3b. windowed small-bulge multishift QR, in three variants of window /
 // shifts / workgroups per CU (qr_ms.inc); the plan's autotuner picks one per
-// matrix size, 48 / 12 / 2 by default.
+// matrix size, 48 / 12 by default.
 // ---------------------------------------------------------------------------
+#define ORCWA_AED_NW QR_AED_NW
 namespace qr_w48 {
 #define ORCWA_QR_W 48
 #define ORCWA_QR_NS 12
 #define ORCWA_QR_WG_PER_CU 2
+#define ORCWA_QR_FUSED
+#define ORCWA_QR_SPLIT
 #include "qr_ms.inc"
+#undef ORCWA_QR_SPLIT
 #undef ORCWA_QR_W
 #undef ORCWA_QR_NS
 #undef ORCWA_QR_WG_PER_CU
@@ -602,7 +646,37 @@ namespace qr_w64 {
 #undef ORCWA_QR_W
 #undef ORCWA_QR_NS
 #undef ORCWA_QR_WG_PER_CU
+#undef ORCWA_QR_FUSED
 }  // namespace qr_w64
+
+__global__ void k_zero_counts(int* a, int n) {
+  for (int i = threadIdx.x; i < n; i += blockDim.x) a[i] = 0;
+}
+
+// The rounds of the two-kernel form.  The host learns how many matrices are
+// left from a counter per round, read back only when about as many sweeps have
+// run as an RCWA matrix takes (n / 12), then every few rounds: a round that
+// finds nothing to do costs two empty launches.
+static void qr_rounds(hipStream_t s, int n, cd* const* A, cd* const* Z, cd* const* X,
+                      cd* const* W, int* counts, int ncounts, int* info, int batch) {
+  const int maxsweep = 40 + 3 * n, strips = 3 * ((n + 63) / 64);
+  const int nc = std::min(ncounts, 1024);
+  int round = 0, check = std::max(2, n / 13);
+  while (true) {
+    const int slot = round % nc;
+    if (slot == 0) hipLaunchKernelGGL(k_zero_counts, dim3(1), dim3(256), 0, s, counts, nc);
+    hipLaunchKernelGGL(qr_w48::k_qr_round, dim3(batch), dim3(qr_w48::SWT), 0, s, n, round, slot, A,
+                       X, W, info, counts, maxsweep);
+    hipLaunchKernelGGL(qr_w48::k_qr_apply, dim3(strips * batch), dim3(256), 0, s, n, batch, A, Z, X, W);
+    ++round;
+    if (round < check) continue;
+    check = round + 2;
+    int left = 0;
+    if (hipMemcpyAsync(&left, counts + slot, sizeof(int), hipMemcpyDeviceToHost, s) != hipSuccess ||
+        hipStreamSynchronize(s) != hipSuccess || left == 0)
+      return;
+  }
+}
 
 // ---------------------------------------------------------------------------
 // 4. eigenvectors of the upper triangular T (ztrevc mathematics, right
@@ -826,7 +900,8 @@ void eig_recover_scatter(hipStream_t s, int n, int m, const int* idx, const cd* 
 
 void zgeev_batched(hipStream_t s, int n, cd* const* A, const cd* const* Aorig, cd* const* W,
                    cd* lam, const EigWorkspace& ws, int* info, double* resid,
-                   cd* const* scratch, int batch, hipEvent_t* ev, double tol, int qr_variant) {
+                   cd* const* scratch, int batch, hipEvent_t* ev, double tol, int qr_variant,
+                   bool host_wait) {
   if (batch <= 0 || n <= 0) return;
   const cd* const* Ac = (const cd* const*)A;
   if (n >= 3) {
@@ -870,7 +945,9 @@ void zgeev_batched(hipStream_t s, int n, cd* const* A, const cd* const* Aorig, c
   if (ev) (void)hipEventRecord(ev[0], s);
   // zero everything below the first subdiagonal (the Householder vectors)
   hipLaunchKernelGGL(k_zero_below_subdiag, dim3(64, batch), dim3(256), 0, s, n, A);
-  switch (qr_variant) {
+  if (host_wait && qr_variant == QR_W48 && qr_split(n, batch))
+    qr_rounds(s, n, A, ws.Z, ws.X, W, reinterpret_cast<int*>(ws.tau), 4 * n * batch, info, batch);
+  else switch (qr_variant) {
     case QR_W32:
       hipLaunchKernelGGL(qr_w32::k_qr_ms, dim3(batch), dim3(256), 0, s, n, A, ws.Z, info,
                          40 + 3 * n);

@@ -75,7 +75,9 @@ void copy_batched(hipStream_t s, long long count, const cd* const* A, cd* const*
 // matrix (Z and X).  Aorig (may equal nullptr) is used for the residual test
 // (accepted when ||Aorig W - W diag(lam)||max / ||Aorig||max <= tol, else
 // ORCWA_STATUS_EIG_RESIDUAL); status bits are or-ed into info[b].  resid[b]
-// receives the relative residual.
+// receives the relative residual.  host_wait: the launcher may wait for the
+// stream (the QR then runs in rounds until no matrix is left; not in a stream
+// capture).
 struct EigWorkspace {
   cd** Z;        // [batch] n*n
   cd** X;        // [batch] n*n
@@ -87,7 +89,7 @@ enum QrVariant { QR_W48 = 0, QR_W32 = 1, QR_W64 = 2, QR_NVARIANTS = 3 };
 void zgeev_batched(hipStream_t s, int n, cd* const* A, const cd* const* Aorig, cd* const* W,
                    cd* lam, const EigWorkspace& ws, int* info, double* resid,
                    cd* const* scratch, int batch, hipEvent_t* phase_events,
-                   double tol = kEigTol, int qr_variant = QR_W48);
+                   double tol = kEigTol, int qr_variant = QR_W48, bool host_wait = true);
 // A[b] = Aorig[b] + diag(1e-11 (i+1) max|Aorig[b]|): the matrix of the
 // reference's recovery solve after a failed residual test
 // (rcwa/MKLEigenSolver.hpp:81-93).

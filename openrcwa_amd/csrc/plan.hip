@@ -1272,7 +1272,8 @@ static int plan_run(orcwa_plan* p, hipStream_t s, bool graph) {
       HIPCHK(record(5));
       zgeev_batched(s, n, A, p->dev<const cd* const*>(ct.pAorig), Wp, p->d_lam, ws,
                     p->d_pinfo + ct.prob_base, p->d_resid + ct.prob_base,
-                    p->dev<cd* const*>(ct.pX), np, nullptr, p->ctx->eig_tol, p->qr_variant);
+                    p->dev<cd* const*>(ct.pX), np, nullptr, p->ctx->eig_tol, p->qr_variant,
+                    !graph);
       if (!graph) {
         const int rc = eig_recover(p, ct, s, recovered);
         if (rc != ORCWA_OK) return rc;

@@ -1,0 +1,31 @@
+"""The QR iteration in rounds (few matrices of 128 rows or more; section 3c of
+csrc/qr_ms.inc) against numpy: sizes at the edges of its 64-line strips and
+48-row windows, with a batch small enough to take it."""
+import numpy as np
+import pytest
+
+from .gpu_helpers import zgeev
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("n,batch", [(128, 1), (129, 2), (191, 3), (192, 1), (257, 5), (338, 2)])
+def test_rounds_match_numpy(gpu_ctx, n, batch):
+    rng = np.random.default_rng(n)
+    a = rng.normal(size=(batch, n, n)) + 1j * rng.normal(size=(batch, n, n))
+    # a graded matrix and one that splits into two blocks, as well as dense ones
+    if batch > 1:
+        a[1] *= np.geomspace(1.0, 1e-3, n)[:, None]
+    if batch > 2:
+        a[2][n // 2:, :n // 2] = 0.0
+    lam, W, resid, info = zgeev(gpu_ctx, a)
+    assert not info.any()
+    # backward error of a QR iteration: a small multiple of n u (2e-14 n here)
+    assert resid.max() <= 2e-14 * n
+    for b in range(batch):
+        ref = np.linalg.eigvals(a[b])
+        # condition numbers of these eigenvalues stay below 1e4
+        tol = 1e4 * 2e-16 * n * np.linalg.norm(a[b], 2)
+        d = np.abs(lam[b][:, None] - ref[None, :])
+        assert d.min(1).max() <= tol and d.min(0).max() <= tol
+        assert np.abs(np.linalg.norm(W[b], axis=0) - 1.0).max() <= 1e-12
