@@ -317,6 +317,215 @@ __global__ __launch_bounds__(256) void k_hess_panel(int n, int i0, int nb, cd* c
   }
 }
 
+// The panel in two launches a column: k_hess_mv forms y = A v in
+// 64-row strips times nch column ranges per matrix (k_hess_panel, one workgroup
+// a matrix, streams it through one compute unit: 52 us a column at n = 450, 177
+// at n = 798), k_hess_col, one workgroup a matrix, finishes Y's column from the
+// partial sums (in the Ytmp region, free during the panel) and forms the next
+// reflector.  Launch order is the only synchronisation.  t and tau of the last
+// reflector wait in Z for the next call.
+constexpr int HC_T = 512;
+__global__ __launch_bounds__(HC_T) void k_hess_col(int n, int i0, int j, int nb, int nch,
+                                                   cd* const* Ap, cd* tau_all, cd* const* Xp,
+                                                   cd* const* Zp) {
+  extern __shared__ cd sm[];
+  cd* sb = sm;          // current column, rows i0+1..n-1
+  __shared__ cd Ts[HB * (HB + 1) / 2];   // T, upper triangular, packed by columns
+  __shared__ cd s_w[HB], s_t[HB], s_row[HB], s_told[HB];
+  __shared__ double sred[HC_T / 64];
+  __shared__ cd s_tau, s_scale;
+  const int mat = blockIdx.x;
+  cd* A = gptr(Ap[mat]);
+  cd* V = gptr(Xp[mat]);
+  cd* Y = V + (long long)n * HB;
+  const cd* P = V + 2LL * n * HB;
+  cd* Tg = V + 3LL * n * HB;
+  cd* tz = gptr(Zp[mat]);
+  cd* tau = tau_all + (long long)mat * n;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int r0 = i0 + 1, c = i0 + j;
+  const long long cc = (long long)c * n;
+  if (j == 0) {
+    for (int e = tid; e < HB * HB; e += HC_T) Tg[e] = mk(0.0, 0.0);
+    // columns outside the panel of V stay zero for the GEMMs
+    for (long long e = (long long)nb * n + tid; e < (long long)HB * n; e += HC_T)
+      V[e] = mk(0.0, 0.0);
+  }
+  if (tid < j) {
+    s_told[tid] = tz[tid];
+    if (j < nb) s_row[tid] = conj(V[c + (long long)tid * n]);
+  }
+  for (int e = tid; e < j * HB; e += HC_T) {
+    const int q = e / HB, r = e % HB;
+    if (r <= q) Ts[q * (q + 1) / 2 + r] = Tg[e];
+  }
+  __syncthreads();
+  // Y(:, j-1) = tau (y - Y(:, 0:j-1) t), and b -= Y(:, 0:j) conj(V(c, 0:j))
+  const cd told = j > 0 ? tau[c - 1] : mk(0.0, 0.0);
+  for (int r = r0 + tid; r < n; r += HC_T) {
+    cd b = j < nb ? A[r + cc] : mk(0.0, 0.0);
+    if (j > 0) {
+      cd y = mk(0.0, 0.0);
+      for (int q = 0; q < nch; ++q) y += P[r + (long long)q * n];
+#pragma unroll 4
+      for (int p = 0; p + 1 < j; ++p) {
+        const cd yp = Y[r + (long long)p * n];
+        y -= yp * s_told[p];
+        b -= yp * s_row[p];
+      }
+      y = told * y;
+      Y[r + (long long)(j - 1) * n] = y;
+      b -= y * s_row[j - 1];
+    }
+    sb[r] = b;
+  }
+  if (j == nb) {
+    if (tid == 0 && i0 + nb == n - 2) {
+      tau[n - 2] = mk(0.0, 0.0);
+      tau[n - 1] = mk(0.0, 0.0);
+    }
+    return;
+  }
+  __syncthreads();
+  if (j > 0) {
+    // b <- (I - V T^H V^H) b
+    for (int p = wave; p < j; p += HC_T / 64) {
+      const cd* vp = V + (long long)p * n;
+      double ar = 0.0, ai = 0.0;
+#pragma unroll 4
+      for (int r = r0 + lane; r < n; r += 64) {
+        const cd z = cmul(vp[r], sb[r]);
+        ar += z.re;
+        ai += z.im;
+      }
+      ar = wave_sum(ar);
+      ai = wave_sum(ai);
+      if (lane == 0) s_w[p] = mk(ar, ai);
+    }
+    __syncthreads();
+    if (tid < j) {
+      cd acc = mk(0.0, 0.0);
+      for (int q = 0; q <= tid; ++q) acc += conj(Ts[tid * (tid + 1) / 2 + q]) * s_w[q];
+      s_t[tid] = acc;
+    }
+    __syncthreads();
+    for (int r = r0 + tid; r < n; r += HC_T) {
+      cd acc = mk(0.0, 0.0);
+#pragma unroll 4
+      for (int p = 0; p < j; ++p) acc += V[r + (long long)p * n] * s_t[p];
+      sb[r] -= acc;
+    }
+    __syncthreads();
+  }
+  // reflector of b(c+1 .. n-1) (zlarfg: H^H x = beta e1)
+  double part = 0.0;
+  for (int r = c + 2 + tid; r < n; r += HC_T) part += norm2(sb[r]);
+  part = wave_sum(part);
+  if (lane == 0) sred[wave] = part;
+  __syncthreads();
+  if (tid == 0) {
+    double xn2 = 0.0;
+    for (int w = 0; w < HC_T / 64; ++w) xn2 += sred[w];
+    const cd alpha = sb[c + 1];
+    cd beta = alpha;
+    if (xn2 == 0.0 && alpha.im == 0.0) {
+      s_tau = mk(0.0, 0.0);
+      s_scale = mk(0.0, 0.0);
+    } else {
+      const double nrm = sqrt(alpha.re * alpha.re + alpha.im * alpha.im + xn2);
+      const double bt = (alpha.re >= 0.0) ? -nrm : nrm;
+      s_tau = mk((bt - alpha.re) / bt, -alpha.im / bt);
+      s_scale = cinv(alpha - mk(bt, 0.0));
+      beta = mk(bt, 0.0);
+    }
+    tau[c] = s_tau;
+    sb[c + 1] = beta;
+  }
+  __syncthreads();
+  const cd t = s_tau, sc = s_scale;
+  cd* Vj = V + (long long)j * n;
+  for (int r = tid; r < n; r += HC_T) {
+    cd v = mk(0.0, 0.0);
+    if (r == c + 1) v = mk(1.0, 0.0);
+    else if (r > c + 1) v = sb[r] * sc;
+    Vj[r] = v;
+    // column c of the reduced matrix: updated entries above the subdiagonal,
+    // beta on it, the reflector below it
+    if (r >= r0) A[r + cc] = (r > c + 1) ? v : sb[r];
+    if (r > c) sb[r] = v;
+  }
+  __syncthreads();
+  // t = V(:, 0:j)^H v
+  for (int p = wave; p < j; p += HC_T / 64) {
+    const cd* vp = V + (long long)p * n;
+    double ar = 0.0, ai = 0.0;
+#pragma unroll 4
+    for (int r = c + 1 + lane; r < n; r += 64) {
+      const cd z = cmul(vp[r], sb[r]);
+      ar += z.re;
+      ai += z.im;
+    }
+    ar = wave_sum(ar);
+    ai = wave_sum(ai);
+    if (lane == 0) s_t[p] = mk(ar, ai);
+  }
+  __syncthreads();
+  // T(0:j, j) = -tau T(0:j, 0:j) t,  T(j, j) = tau
+  if (tid < j) {
+    cd acc = mk(0.0, 0.0);
+    for (int q = tid; q < j; ++q) acc += Ts[q * (q + 1) / 2 + tid] * s_t[q];
+    Tg[tid + j * HB] = -(t * acc);
+    tz[tid] = s_t[tid];
+  }
+  if (tid == j) Tg[j + j * HB] = t;
+}
+
+__global__ __launch_bounds__(256) void k_hess_mv(int n, int i0, int j, int cw, cd* const* Ap,
+                                                 cd* const* Xp) {
+  __shared__ cd sv[256];
+  __shared__ cd red[4][64];
+  const cd* A = gptr(Ap[blockIdx.z]);
+  cd* V = gptr(Xp[blockIdx.z]);
+  cd* P = V + 2LL * n * HB;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int r = i0 + 1 + 64 * (int)blockIdx.x + lane;
+  const int q0 = i0 + j + 1 + (int)blockIdx.y * cw, q1 = min(n, q0 + cw);
+  if (tid < q1 - q0) sv[tid] = V[q0 + tid + (long long)j * n];
+  __syncthreads();
+  cd y = mk(0.0, 0.0);
+  if (r < n) {
+#pragma unroll 8
+    for (int q = q0 + wave; q < q1; q += 4) y += A[r + (long long)q * n] * sv[q - q0];
+  }
+  red[wave][lane] = y;
+  __syncthreads();
+  if (wave == 0 && r < n)
+    P[r + (long long)blockIdx.y * n] = red[0][lane] + red[1][lane] + red[2][lane] + red[3][lane];
+}
+
+// Which panel kernel: the one workgroup a matrix only where matrices are small
+// and many.  Time of a pillar batch with the split panel / without, ms: n = 162,
+// 600 matrices 69.6 / 67.5; n = 242, 240: 74.5 / 74.8, 400: 91.9 / 93.5, 760:
+// 149 / 144; n = 450, 4: 121 / 136, 256: 235 / 262, 1280: 885 / 903; n = 722,
+// 3: 235 / 322.
+static bool hess_split(int n, int batch) { return n >= 300 || batch <= 512; }
+
+static void hess_panel_split(hipStream_t s, int n, int i0, int nb, cd* const* A, cd* tau,
+                           cd* const* X, cd* const* Z, int batch) {
+  const int strips = (n - i0 - 1 + 63) / 64;
+  // column ranges: about 768 workgroups in all, at most 256 and at least 16
+  // columns each
+  int nch = std::min(768 / (strips * batch), (n - i0 - 1) / 16);
+  nch = std::min(std::max({nch, 1, (n - i0 - 1 + 255) / 256}), HB);
+  const int cw = (n - i0 - 1 + nch - 1) / nch;
+  for (int j = 0; j <= nb; ++j) {
+    hipLaunchKernelGGL(k_hess_col, dim3(batch), dim3(HC_T), n * sizeof(cd), s, n, i0, j, nb, nch,
+                       A, tau, X, Z);
+    if (j < nb)
+      hipLaunchKernelGGL(k_hess_mv, dim3(strips, nch, batch), dim3(256), 0, s, n, i0, j, cw, A, X);
+  }
+}
+
 static void hess_blocked(hipStream_t s, int n, cd* const* A, cd* tau, cd* const* X,
                          cd* const* Z, int batch) {
   const cd one = mk(1.0, 0.0), mone = mk(-1.0, 0.0), zero = mk(0.0, 0.0);
@@ -328,8 +537,11 @@ static void hess_blocked(hipStream_t s, int n, cd* const* A, cd* tau, cd* const*
   for (int i0 = 0; i0 + 2 < n; i0 += HB) {
     const int nb = std::min(HB, n - 2 - i0);
     const int top = i0 + 1, m = n - i0 - 1, nt = n - i0 - nb;
-    hipLaunchKernelGGL(k_hess_panel, dim3(batch), dim3(256), 2 * n * sizeof(cd), s, n, i0, nb,
-                       A, tau, X);
+    if (hess_split(n, batch))
+      hess_panel_split(s, n, i0, nb, A, tau, X, Z, batch);
+    else
+      hipLaunchKernelGGL(k_hess_panel, dim3(batch), dim3(256), 2 * n * sizeof(cd), s, n, i0, nb,
+                         A, tau, X);
     // Ytmp(0:top) = A(0:top, i0+1:n) V(i0+1:n, :);  Y(0:top) = Ytmp T
     zgemm_batched(s, top, nb, m, one, Ac, (long long)top * n, 1, n, 0, Xc, oV + top, 1, n, 0,
                   zero, X, oYt, 1, n, batch);
