@@ -20,7 +20,6 @@
 namespace orcwa {
 
 typedef double v4d __attribute__((ext_vector_type(4)));
-typedef double v2d __attribute__((ext_vector_type(2)));
 
 static constexpr double kUlp = DBL_EPSILON;
 static constexpr double kSafmin = DBL_MIN;

@@ -82,6 +82,21 @@ __device__ __forceinline__ T* gptr(T* p) {
   return (T*)((__attribute__((address_space(1))) T*)(unsigned long long)p);
 }
 
+typedef double v2d __attribute__((ext_vector_type(2)));
+
+// 16-byte LDS accesses (cd alone is only 8-byte aligned to the compiler, which
+// then moves it as two 8-byte halves, each with half the banks in conflict)
+__device__ __forceinline__ cd lds_ld(const cd* p) {
+  const v2d v = *reinterpret_cast<const v2d*>(p);
+  return mk(v.x, v.y);
+}
+__device__ __forceinline__ void lds_st(cd* p, cd z) {
+  v2d v;
+  v.x = z.re;
+  v.y = z.im;
+  *reinterpret_cast<v2d*>(p) = v;
+}
+
 // wavefront (64-lane) helpers
 __device__ inline double wave_sum(double v) {
   for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
