@@ -737,120 +737,175 @@ __global__ __launch_bounds__(256) void k_getf2_panel(int n, int k0, int nb, cd* 
 }
 
 // The same panel factorization held in registers, for panels of at most
-// GF_T rows: thread t owns row k0 + t of the nb <= NB panel columns.  Per
-// column: the pivot search (wave shuffles, one barrier), the row exchange and
-// the pivot-row broadcast through LDS (one barrier), then the scaling and the
-// rank-1 update of the thread's own row; the panel is read and written once.
+// GF_T rows: thread t owns one row of the nb <= NB panel columns.  The rows do
+// not move: a thread keeps the position that the interchanges give its row and
+// stores it there at the end.  Per column one barrier: every wave reduces its
+// pivot candidate with DPP moves (no LDS round trips) and puts that row in LDS
+// beside the others', so that after the barrier each thread finds the winner
+// and reads its row from the wave's buffer.  (Rows exchanged through LDS, two
+// barriers and shuffled reductions took 2.4 us a column at n = 450, this 1.5.)
 // The column steps are instantiated one by one (template recursion) so that
 // every register index is a constant.
-constexpr int GF_T = 512;
+constexpr int GF_T = 512, GF_T2 = 1024, NB2 = 16;
 
+// T threads (rows), WB panel columns: 512 x 32, or 1024 x 16 (a thread's row
+// then fits the 128 registers it has)
+template <int T, int WB>
 struct GetrfRegState {
-  cd (*s_row)[2][NB];       // [parity][2][NB]: the pivot row, the displaced row c
-  double (*s_wv)[GF_T / 64];
-  int (*s_wi)[GF_T / 64];
-  int n, k0, nb, r, t, lane, wave, b;
-  bool live;
+  cd (*s_row)[T / 64][WB];       // [parity][wave]: the wave's candidate row
+  double (*s_wv)[T / 64];
+  int (*s_wp)[T / 64];
+  int n, k0, nb, lane, wave, b;
+  int pos;                          // position of this thread's row (n: no row)
   int* ipiv;
   int* info;
   const int* info_map;
 };
 
-template <int J>
-__device__ __forceinline__ void getrf_reg_step(const GetrfRegState& S, cd (&a)[NB]) {
-  if constexpr (J < NB) {
+// value of lane (lane + shift inside the row / row broadcasts) of a double
+template <int CTRL>
+__device__ __forceinline__ double dpp_move(double v) {
+  union { double d; int i[2]; } u;
+  u.d = v;
+  u.i[0] = __builtin_amdgcn_update_dpp(u.i[0], u.i[0], CTRL, 0xf, 0xf, false);
+  u.i[1] = __builtin_amdgcn_update_dpp(u.i[1], u.i[1], CTRL, 0xf, 0xf, false);
+  return u.d;
+}
+__device__ __forceinline__ double lane_double(double v, int lane) {
+  union { double d; int i[2]; } u;
+  u.d = v;
+  u.i[0] = __builtin_amdgcn_readlane(u.i[0], lane);
+  u.i[1] = __builtin_amdgcn_readlane(u.i[1], lane);
+  return u.d;
+}
+// maximum over the first 16 lanes, and over the wave, in every lane (lanes
+// without a source keep their own)
+__device__ __forceinline__ double dpp_row_reduce(double v) {
+  v = fmax(v, dpp_move<0x111>(v));   // row_shr:1
+  v = fmax(v, dpp_move<0x112>(v));   // row_shr:2
+  v = fmax(v, dpp_move<0x114>(v));   // row_shr:4
+  return fmax(v, dpp_move<0x118>(v));   // row_shr:8
+}
+__device__ __forceinline__ double dpp_row_max(double v) {
+  return lane_double(dpp_row_reduce(v), 15);
+}
+__device__ __forceinline__ double dpp_wave_max(double v) {
+  v = dpp_row_reduce(v);
+  v = fmax(v, dpp_move<0x142>(v));   // row_bcast:15
+  v = fmax(v, dpp_move<0x143>(v));   // row_bcast:31
+  return lane_double(v, 63);
+}
+
+// 1 / z: conj(z) times the Newton-refined reciprocal of |z|^2 (2 ulp; a tenth
+// of the instructions of the division), Smith's division near the ends of the
+// range
+__device__ __forceinline__ cd pivot_inv(cd z) {
+  const double n2 = norm2(z);
+  if (n2 > 1e-280 && n2 < 1e280) {
+    double y = __builtin_amdgcn_rcp(n2);
+    y = fma(y, fma(-n2, y, 1.0), y);
+    y = fma(y, fma(-n2, y, 1.0), y);
+    return mk(z.re * y, -z.im * y);
+  }
+  return cinv(z);
+}
+
+template <int J, int T, int WB>
+__device__ __forceinline__ void getrf_reg_step(GetrfRegState<T, WB>& S, cd (&a)[WB]) {
+  if constexpr (J < WB) {
     if (J < S.nb) {
       const int c = S.k0 + J, par = J & 1;
-      const int r = S.r;
-      // pivot: max cabs1 over rows c..n-1, the first index on ties
-      double v = (S.live && S.t >= J) ? cabs1(a[J]) : -1.0;
-      int vi = r;
+      // the wave's pivot: max cabs1 over its rows at positions c..n-1 (-1: it
+      // has none; a NaN counts as 0), the lowest position on ties
+      const bool in = S.pos >= c && S.pos < S.n;
+      const double v0 = cabs1(a[J]);
+      const double v = in ? (v0 == v0 ? v0 : 0.0) : -1.0;
+      const double best = dpp_wave_max(v);
+      if (best >= 0.0) {
+        unsigned long long who = __ballot(v == best);
+        int bl = __ffsll(who) - 1, bp = __builtin_amdgcn_readlane(S.pos, bl);
+        for (who &= who - 1; who; who &= who - 1) {
+          const int l = __ffsll(who) - 1, p = __builtin_amdgcn_readlane(S.pos, l);
+          if (p < bp) {
+            bp = p;
+            bl = l;
+          }
+        }
+        if (S.lane == bl) {
+          S.s_wp[par][S.wave] = bp;
 #pragma unroll
-      for (int off = 32; off > 0; off >>= 1) {
-        const double ov = __shfl_xor(v, off, 64);
-        const int oi = __shfl_xor(vi, off, 64);
-        if (ov > v || (ov == v && oi < vi)) {
-          v = ov;
-          vi = oi;
+          for (int jj = J; jj < WB; ++jj) lds_st(&S.s_row[par][S.wave][jj], a[jj]);
         }
       }
-      if (S.lane == 0) {
-        S.s_wv[par][S.wave] = v;
-        S.s_wi[par][S.wave] = vi;
-      }
+      if (S.lane == 0) S.s_wv[par][S.wave] = best;
       __syncthreads();
-      double bv = S.s_wv[par][0];
-      int bi = S.s_wi[par][0];
-#pragma unroll
-      for (int w = 1; w < GF_T / 64; ++w) {
-        const double ov = S.s_wv[par][w];
-        const int oi = S.s_wi[par][w];
-        if (ov > bv || (ov == bv && oi < bi)) {
-          bv = ov;
-          bi = oi;
+      // the winner among the waves' candidates, lane w holding wave w's
+      const double cv = S.lane < T / 64 ? S.s_wv[par][S.lane] : -1.0;
+      const int cp = S.s_wp[par][S.lane & (T / 64 - 1)];
+      const double top = dpp_row_max(cv);
+      unsigned long long won = __ballot(cv == top);
+      int bw = __ffsll(won) - 1, bi = __builtin_amdgcn_readlane(cp, bw);
+      for (won &= won - 1; won; won &= won - 1) {
+        const int w = __ffsll(won) - 1, q = __builtin_amdgcn_readlane(cp, w);
+        if (q < bi) {
+          bi = q;
+          bw = w;
         }
       }
-      // rows c and bi trade places; s_row[0] becomes row c for every thread
-      const int put = (r == bi) ? 0 : ((r == c && bi != c) ? 1 : -1);
-      if (put >= 0) {
-#pragma unroll
-        for (int jj = 0; jj < NB; ++jj) S.s_row[par][put][jj] = a[jj];
-      }
-      __syncthreads();
-      const int take = (bi == c) ? -1 : ((r == c) ? 0 : ((r == bi) ? 1 : -1));
-      if (take >= 0) {
-#pragma unroll
-        for (int jj = 0; jj < NB; ++jj) a[jj] = S.s_row[par][take][jj];
-      }
-      const cd pv = S.s_row[par][0][J];
+      const cd* prow = S.s_row[par][bw];
+      const cd pv = lds_ld(&prow[J]);
       const bool zero = (pv.re == 0.0 && pv.im == 0.0);
-      if (S.t == 0) {
+      if (threadIdx.x == 0) {
         S.ipiv[(long long)S.b * S.n + c] = bi;
         if (zero) atomicOr(&S.info[S.info_map ? S.info_map[S.b] : S.b], ORCWA_STATUS_SINGULAR);
       }
-      if (S.live && r > c) {
-        a[J] = zero ? mk(0.0, 0.0) : a[J] * cinv(pv);
+      const cd inv = pivot_inv(pv);
+      // rows c and bi trade positions
+      S.pos = S.pos == bi ? c : (S.pos == c ? bi : S.pos);
+      if (S.pos > c && S.pos < S.n) {
+        a[J] = zero ? mk(0.0, 0.0) : a[J] * inv;
 #pragma unroll
-        for (int jj = J + 1; jj < NB; ++jj) a[jj] -= a[J] * S.s_row[par][0][jj];
+        for (int jj = J + 1; jj < WB; ++jj) a[jj] = cfnma(a[jj], a[J], lds_ld(&prow[jj]));
       }
-      // (s_row and the wave maxima alternate by column parity: the next
-      // column writes the other half, and the one after writes this half
-      // only after every thread has passed the next column's two barriers)
-      getrf_reg_step<J + 1>(S, a);
+      // (the candidates alternate by column parity: the next column writes the
+      // other half, and the one after writes this half only after every thread
+      // has passed the next column's barrier)
+      getrf_reg_step<J + 1, T, WB>(S, a);
     }
   }
 }
 
-__global__ __launch_bounds__(GF_T) void k_getf2_reg(int n, int k0, int nb, cd* const* Ap,
+template <int T, int WB>
+__global__ __launch_bounds__(T) void k_getf2_reg(int n, int k0, int nb, cd* const* Ap,
                                                     int* ipiv, int* info, const int* info_map) {
-  __shared__ cd s_row[2][2][NB];
-  __shared__ double s_wv[2][GF_T / 64];
-  __shared__ int s_wi[2][GF_T / 64];
-  GetrfRegState S;
+  __shared__ alignas(16) cd s_row[2][T / 64][WB];
+  __shared__ double s_wv[2][T / 64];
+  __shared__ int s_wp[2][T / 64];
+  GetrfRegState<T, WB> S;
   S.s_row = s_row;
   S.s_wv = s_wv;
-  S.s_wi = s_wi;
+  S.s_wp = s_wp;
   S.n = n;
   S.k0 = k0;
   S.nb = nb;
   S.b = blockIdx.x;
-  S.t = threadIdx.x;
-  S.lane = S.t & 63;
-  S.wave = S.t >> 6;
-  S.r = k0 + S.t;
-  S.live = S.r < n;
+  S.lane = threadIdx.x & 63;
+  S.wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int r = k0 + threadIdx.x;
+  const bool live = r < n;
+  S.pos = live ? r : n;
   S.ipiv = ipiv;
   S.info = info;
   S.info_map = info_map;
   cd* __restrict__ A = gptr(Ap[S.b]);
-  cd a[NB];
+  cd a[WB];
 #pragma unroll
-  for (int j = 0; j < NB; ++j)
-    a[j] = (S.live && j < nb) ? A[S.r + (long long)(k0 + j) * n] : mk(0.0, 0.0);
-  getrf_reg_step<0>(S, a);
+  for (int j = 0; j < WB; ++j)
+    a[j] = (live && j < nb) ? A[r + (long long)(k0 + j) * n] : mk(0.0, 0.0);
+  getrf_reg_step<0, T, WB>(S, a);
 #pragma unroll
-  for (int j = 0; j < NB; ++j)
-    if (S.live && j < nb) A[S.r + (long long)(k0 + j) * n] = a[j];
+  for (int j = 0; j < WB; ++j)
+    if (live && j < nb) A[S.pos + (long long)(k0 + j) * n] = a[j];
 }
 
 // Apply row swaps ipiv[k0..k0+nb) (in order) to columns [c0, c1) of an
@@ -874,48 +929,52 @@ __global__ void k_laswp(int n, int ncols_total, int k0, int nb, int c0, int c1, 
 }
 
 // The interchanges of one panel (rows k0..k0+nb-1 with their pivot rows,
-// applied in order) as a single gather: thread 0 composes them on the <= 2 nb
-// rows they touch (slot s holds row R[s]; after the swaps it holds the
-// original row R[src[s]]); the workgroup then stages those rows of its 16
-// columns in LDS and writes back the moved ones.  Columns [c0, c1).
+// applied in order) as a single gather on the columns left and right of it: one
+// wave composes them on the <= 2 nb rows they touch (lane s holds row R; after
+// the swaps it holds the original row of lane src), in registers (in LDS by one
+// thread it took most of the kernel's 21 us); the workgroup then stages those
+// rows of its 16 columns in LDS and writes back the moved ones.
 constexpr int LASWP_MAXS = 64, LASWP_NC = 16;
-__global__ __launch_bounds__(256) void k_laswp_panel(int n, int k0, int nb, int c0, int c1,
-                                                     cd* const* Ap, const int* ipiv) {
-  __shared__ int R[LASWP_MAXS], src[LASWP_MAXS];
+static_assert(2 * NB <= LASWP_MAXS, "one lane per touched row");
+__global__ __launch_bounds__(256) void k_laswp_panel(int n, int k0, int nb, cd* const* Ap,
+                                                     const int* ipiv) {
+  __shared__ int s_R[LASWP_MAXS], s_src[LASWP_MAXS];
   __shared__ int s_ns;
-  __shared__ cd tile[LASWP_MAXS][LASWP_NC];
+  __shared__ alignas(16) cd tile[LASWP_MAXS][LASWP_NC];
   const int b = blockIdx.y;
   const int* pv = ipiv + (long long)b * n;
-  if (threadIdx.x == 0) {
-    int ns = nb;
-    for (int j = 0; j < nb; ++j) { R[j] = k0 + j; src[j] = j; }
+  if (threadIdx.x < 64) {
+    const int lane = threadIdx.x;
+    const int piv = lane < nb ? pv[k0 + lane] : -1;
+    int R = lane < nb ? k0 + lane : -1, src = lane, ns = nb;
     for (int j = 0; j < nb; ++j) {
-      const int p = pv[k0 + j];
-      int sp = -1;
-      if (p < k0 + nb) {
-        sp = p - k0;
-      } else {
-        for (int t = nb; t < ns; ++t)
-          if (R[t] == p) { sp = t; break; }
-        if (sp < 0) { sp = ns; R[ns] = p; src[ns] = ns; ++ns; }
+      const int p = __builtin_amdgcn_readlane(piv, j);
+      const unsigned long long m = __ballot(R == p);
+      int sp = ns;
+      if (m) sp = __ffsll(m) - 1;
+      else {
+        if (lane == ns) R = p;
+        ++ns;
       }
-      const int t = src[j];
-      src[j] = src[sp];
-      src[sp] = t;
+      const int sj = __builtin_amdgcn_readlane(src, j), ss = __builtin_amdgcn_readlane(src, sp);
+      if (lane == j) src = ss;
+      if (lane == sp) src = sj;
     }
-    s_ns = ns;
+    s_R[lane] = R;
+    s_src[lane] = src;
+    if (lane == 0) s_ns = ns;
   }
   __syncthreads();
   const int ns = s_ns;
   const int c = threadIdx.x % LASWP_NC, sg = threadIdx.x / LASWP_NC;
-  const int col = c0 + blockIdx.x * LASWP_NC + c;
+  const int idx = blockIdx.x * LASWP_NC + c, col = idx < k0 ? idx : idx + nb;
   cd* __restrict__ A = gptr(Ap[b]) + (long long)col * n;
-  if (col < c1)
-    for (int t = sg; t < ns; t += 256 / LASWP_NC) tile[t][c] = A[R[t]];
+  if (col < n)
+    for (int t = sg; t < ns; t += 256 / LASWP_NC) lds_st(&tile[t][c], A[s_R[t]]);
   __syncthreads();
-  if (col < c1)
+  if (col < n)
     for (int t = sg; t < ns; t += 256 / LASWP_NC)
-      if (src[t] != t) A[R[t]] = tile[src[t]][c];
+      if (s_src[t] != t) A[s_R[t]] = lds_ld(&tile[s_src[t]][c]);
 }
 
 // perm[r] = the original row that ends in row r after all n interchanges
@@ -969,36 +1028,40 @@ __global__ __launch_bounds__(256) void k_apply_perm(int n, int nrhs, int ncw, co
 // thread; the block moves between HBM and registers through LDS in slabs of
 // TR_SLAB rows, so that consecutive threads touch consecutive rows of a
 // column (a column's 32-row segment is 512 contiguous bytes; read directly,
-// the lanes of a wave would each touch another column).
+// the lanes of a wave would each touch another column).  All slabs are loaded
+// before the first is staged: one memory latency instead of four.
 constexpr int TR_SLAB = 8;
-template <bool UNIT_LOWER>
-__global__ __launch_bounds__(256) void k_trsm_block(int n, int k0, int nb, int c0, int ncols,
+template <bool UNIT_LOWER, int TPB>
+__global__ __launch_bounds__(TPB) void k_trsm_block(int n, int k0, int nb, int c0, int ncols,
                                                     const cd* const* Lp, cd* const* Xp) {
-  __shared__ cd sT[NB][NB];
-  __shared__ cd sX[256][TR_SLAB + 1];
+  __shared__ alignas(16) cd sT[NB][NB];
+  __shared__ alignas(16) cd sX[TPB][TR_SLAB + 1];
   const int b = blockIdx.y;
   const cd* __restrict__ Lm = gptr(Lp[b]);
   cd* __restrict__ X = gptr(Xp[b]);
   const int tid = threadIdx.x;
+  const int cb = blockIdx.x * TPB;   // this workgroup's first column (from c0)
+  const int rr0 = tid % TR_SLAB;
+  cd r[NB];
+#pragma unroll
+  for (int e = 0; e < NB; ++e) {
+    const int cc = tid / TR_SLAB + (TPB / TR_SLAB) * (e % TR_SLAB), row = TR_SLAB * (e / TR_SLAB) + rr0;
+    r[e] = (cb + cc < ncols && row < nb) ? X[(long long)(c0 + cb + cc) * n + k0 + row]
+                                         : mk(0.0, 0.0);
+  }
   // (zero outside nb x nb, so the unrolled products below need no guard)
-  for (int e = tid; e < NB * NB; e += 256) {
+  for (int e = tid; e < NB * NB; e += TPB) {
     const int i = e % NB, j = e / NB;
     sT[i][j] = (i < nb && j < nb) ? Lm[(k0 + i) + (long long)(k0 + j) * n] : mk(0.0, 0.0);
   }
-  const int cb = blockIdx.x * 256;   // this workgroup's first column (from c0)
-  cd r[NB];
 #pragma unroll
   for (int q = 0; q < NB / TR_SLAB; ++q) {
 #pragma unroll
-    for (int i = 0; i < TR_SLAB; ++i) {
-      const int e = tid + 256 * i, cc = e / TR_SLAB, rr = e % TR_SLAB;
-      const int row = TR_SLAB * q + rr;
-      sX[cc][rr] = (cb + cc < ncols && row < nb) ? X[(long long)(c0 + cb + cc) * n + k0 + row]
-                                                 : mk(0.0, 0.0);
-    }
+    for (int i = 0; i < TR_SLAB; ++i)
+      lds_st(&sX[tid / TR_SLAB + (TPB / TR_SLAB) * i][rr0], r[TR_SLAB * q + i]);
     __syncthreads();
 #pragma unroll
-    for (int rr = 0; rr < TR_SLAB; ++rr) r[TR_SLAB * q + rr] = sX[tid][rr];
+    for (int rr = 0; rr < TR_SLAB; ++rr) r[TR_SLAB * q + rr] = lds_ld(&sX[tid][rr]);
     __syncthreads();
   }
   // (columns past ncols hold zeros and are not stored)
@@ -1008,7 +1071,7 @@ __global__ __launch_bounds__(256) void k_trsm_block(int n, int k0, int nb, int c
       if (i < nb) {
 #pragma unroll
         for (int k = 0; k < NB; ++k)
-          if (k < i) r[i] -= sT[i][k] * r[k];
+          if (k < i) r[i] = cfnma(r[i], lds_ld(&sT[i][k]), r[k]);
       }
     }
   } else {  // upper, non-unit
@@ -1016,7 +1079,7 @@ __global__ __launch_bounds__(256) void k_trsm_block(int n, int k0, int nb, int c
     for (int ii = NB - 1; ii >= 0; --ii) {
       if (ii < nb) {
 #pragma unroll
-        for (int k = ii + 1; k < NB; ++k) r[ii] -= sT[ii][k] * r[k];
+        for (int k = ii + 1; k < NB; ++k) r[ii] = cfnma(r[ii], lds_ld(&sT[ii][k]), r[k]);
         cd d = sT[ii][ii];
         if (d.re != 0.0 || d.im != 0.0) r[ii] = cdiv(r[ii], d);
       }
@@ -1025,40 +1088,58 @@ __global__ __launch_bounds__(256) void k_trsm_block(int n, int k0, int nb, int c
 #pragma unroll
   for (int q = 0; q < NB / TR_SLAB; ++q) {
 #pragma unroll
-    for (int rr = 0; rr < TR_SLAB; ++rr) sX[tid][rr] = r[TR_SLAB * q + rr];
+    for (int rr = 0; rr < TR_SLAB; ++rr) lds_st(&sX[tid][rr], r[TR_SLAB * q + rr]);
     __syncthreads();
 #pragma unroll
     for (int i = 0; i < TR_SLAB; ++i) {
-      const int e = tid + 256 * i, cc = e / TR_SLAB, rr = e % TR_SLAB;
-      const int row = TR_SLAB * q + rr;
-      if (cb + cc < ncols && row < nb) X[(long long)(c0 + cb + cc) * n + k0 + row] = sX[cc][rr];
+      const int cc = tid / TR_SLAB + (TPB / TR_SLAB) * i, row = TR_SLAB * q + rr0;
+      if (cb + cc < ncols && row < nb)
+        X[(long long)(c0 + cb + cc) * n + k0 + row] = lds_ld(&sX[cc][rr0]);
     }
     __syncthreads();
   }
+}
+
+// 256 columns a workgroup where that fills the chip, else 64 (one wave: more
+// workgroups, no waiting between waves)
+template <bool UNIT_LOWER>
+static void trsm_block(hipStream_t s, int n, int k0, int nb, int c0, int ncols,
+                       const cd* const* L, cd* const* X, int batch) {
+  if ((long long)((ncols + 255) / 256) * batch >= 512)
+    hipLaunchKernelGGL((k_trsm_block<UNIT_LOWER, 256>), dim3((ncols + 255) / 256, batch), dim3(256),
+                       0, s, n, k0, nb, c0, ncols, L, X);
+  else
+    hipLaunchKernelGGL((k_trsm_block<UNIT_LOWER, 64>), dim3((ncols + 63) / 64, batch), dim3(64), 0,
+                       s, n, k0, nb, c0, ncols, L, X);
 }
 
 void zgetrf_batched(hipStream_t s, int n, cd* const* A, int* ipiv, int* info,
                     const int* info_map, int batch) {
   if (n <= 0 || batch <= 0) return;
   const cd* const* Ac = (const cd* const*)A;
-  for (int k0 = 0; k0 < n; k0 += NB) {
-    const int nb = (n - k0 < NB) ? (n - k0) : NB;
-    if (n - k0 <= GF_T)
-      hipLaunchKernelGGL(k_getf2_reg, dim3(batch), dim3(GF_T), 0, s, n, k0, nb, A, ipiv, info,
-                         info_map);
+  for (int k0 = 0, nb; k0 < n; k0 += nb) {
+    const int rows = n - k0;
+    // panels of 513 to 1024 rows are kept in registers 16 columns at a time
+    // where launches, not the trailing update's traffic (twice the passes),
+    // take the time: one n = 798 stack 229 -> 219 ms
+    const bool half = rows > GF_T && rows <= GF_T2 && batch <= 64;
+    nb = std::min(half ? NB2 : NB, rows);
+    if (rows <= GF_T)
+      hipLaunchKernelGGL((k_getf2_reg<GF_T, NB>), dim3(batch), dim3(GF_T), 0, s, n, k0, nb, A, ipiv,
+                         info, info_map);
+    else if (half)
+      hipLaunchKernelGGL((k_getf2_reg<GF_T2, NB2>), dim3(batch), dim3(GF_T2), 0, s, n, k0, nb, A,
+                         ipiv, info, info_map);
     else
       hipLaunchKernelGGL(k_getf2_panel, dim3(batch), dim3(256), 0, s, n, k0, nb, A, ipiv, info,
                          info_map);
     // swaps on the columns left and right of the panel
-    if (k0 > 0)
-      hipLaunchKernelGGL(k_laswp_panel, dim3((k0 + LASWP_NC - 1) / LASWP_NC, batch), dim3(256), 0,
-                         s, n, k0, nb, 0, k0, A, (const int*)ipiv);
+    if (n > nb)
+      hipLaunchKernelGGL(k_laswp_panel, dim3((n - nb + LASWP_NC - 1) / LASWP_NC, batch), dim3(256),
+                         0, s, n, k0, nb, A, (const int*)ipiv);
     const int rest = n - k0 - nb;
     if (rest > 0) {
-      hipLaunchKernelGGL(k_laswp_panel, dim3((rest + LASWP_NC - 1) / LASWP_NC, batch), dim3(256),
-                         0, s, n, k0, nb, k0 + nb, n, A, (const int*)ipiv);
-      hipLaunchKernelGGL(k_trsm_block<true>, dim3((rest + 255) / 256, batch), dim3(256), 0, s, n,
-                         k0, nb, k0 + nb, rest, Ac, A);
+      trsm_block<true>(s, n, k0, nb, k0 + nb, rest, Ac, A, batch);
       // A22 -= L21 * U12
       zgemm_batched(s, rest, rest, nb, mk(-1.0, 0.0), Ac, (long long)(k0 + nb) + (long long)k0 * n,
                     1, n, 0, Ac, (long long)k0 + (long long)(k0 + nb) * n, 1, n, 0, mk(1.0, 0.0), A,
@@ -1099,8 +1180,7 @@ void zgetrs_batched(hipStream_t s, int n, int nrhs, const cd* const* LU, const i
     const int oe = std::min(n, o0 + OB);
     for (int k0 = o0; k0 < oe; k0 += NB) {
       const int nb = std::min(NB, oe - k0);
-      hipLaunchKernelGGL(k_trsm_block<true>, dim3((nrhs + 255) / 256, batch), dim3(256), 0, s, n,
-                         k0, nb, 0, nrhs, LU, B);
+      trsm_block<true>(s, n, k0, nb, 0, nrhs, LU, B, batch);
       const int rin = oe - k0 - nb;
       if (rin > 0)
         zgemm_batched(s, rin, nrhs, nb, mone, LU, (long long)(k0 + nb) + (long long)k0 * n, 1, n,
@@ -1117,8 +1197,7 @@ void zgetrs_batched(hipStream_t s, int n, int nrhs, const cd* const* LU, const i
     const int nib = (oe - o0 + NB - 1) / NB;
     for (int ib = nib - 1; ib >= 0; --ib) {
       const int k0 = o0 + ib * NB, nb = std::min(NB, oe - k0);
-      hipLaunchKernelGGL(k_trsm_block<false>, dim3((nrhs + 255) / 256, batch), dim3(256), 0, s, n,
-                         k0, nb, 0, nrhs, LU, B);
+      trsm_block<false>(s, n, k0, nb, 0, nrhs, LU, B, batch);
       if (k0 > o0)
         zgemm_batched(s, k0 - o0, nrhs, nb, mone, LU, (long long)o0 + (long long)k0 * n, 1, n, 0,
                       Bc, (long long)k0, 1, n, 0, one, B, (long long)o0, 1, n, batch);

@@ -36,6 +36,17 @@ __host__ __device__ inline cd mulc(cd a, cd b) {
 __host__ __device__ inline cd cmul(cd a, cd b) {
   return mk(a.re * b.re + a.im * b.im, a.re * b.im - a.im * b.re);
 }
+// acc + a b, acc - a b and acc + conj(a) b in four fused operations (written
+// with the operators: two products of two operations and two sums)
+__host__ __device__ inline cd cfma(cd acc, cd a, cd b) {
+  return mk(fma(a.re, b.re, fma(-a.im, b.im, acc.re)), fma(a.re, b.im, fma(a.im, b.re, acc.im)));
+}
+__host__ __device__ inline cd cfnma(cd acc, cd a, cd b) {
+  return mk(fma(-a.re, b.re, fma(a.im, b.im, acc.re)), fma(-a.re, b.im, fma(-a.im, b.re, acc.im)));
+}
+__host__ __device__ inline cd cfmac(cd acc, cd a, cd b) {
+  return mk(fma(a.re, b.re, fma(a.im, b.im, acc.re)), fma(a.re, b.im, fma(-a.im, b.re, acc.im)));
+}
 __host__ __device__ inline cd cdiv(cd a, cd b) {
   // Smith's algorithm
   if (fabs(b.re) >= fabs(b.im)) {
