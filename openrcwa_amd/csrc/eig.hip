@@ -144,7 +144,7 @@ __global__ __launch_bounds__(256) void k_hess(int n, cd* const* Ap, cd* tau_all)
 
 // ---------------------------------------------------------------------------
 // 1b. blocked Hessenberg reduction (zgehrd / zlahr2 order) for large n.
-//     Per block of HB columns [i0, i0+nb): k_hess_panel reduces the panel
+//     Per block of HB columns [i0, i0+nb): hess_panel reduces the panel
 //     columns one by one, keeping the rest of the matrix at its block-start
 //     value and representing the block's transformation Q_b = I - V T V^H by
 //     V (explicit, n x HB), T (HB x HB) and Y = A V T (rows i0+1..n-1); the
@@ -160,166 +160,10 @@ __global__ __launch_bounds__(256) void k_hess(int n, cd* const* Ap, cd* tau_all)
 // ---------------------------------------------------------------------------
 constexpr int HB = 32;
 
-__global__ __launch_bounds__(256) void k_hess_panel(int n, int i0, int nb, cd* const* Ap,
-                                                    cd* tau_all, cd* const* Xp) {
-  extern __shared__ cd sm[];
-  cd* sb = sm;          // current column, rows i0+1..n-1
-  cd* sv = sm + n;      // current reflector
-  // T of the panel's block reflector, upper triangular, packed by columns:
-  // T(r, c) at c (c + 1) / 2 + r, r <= c
-  __shared__ cd Ts[HB * (HB + 1) / 2];
-  __shared__ cd s_w[HB], s_t[HB], s_row[HB];
-  __shared__ double sred[4];
-  __shared__ cd s_tau, s_scale;
-
-  const int mat = blockIdx.x;
-  cd* __restrict__ A = gptr(Ap[mat]);
-  cd* __restrict__ V = gptr(Xp[mat]);
-  cd* __restrict__ Y = V + (long long)n * HB;
-  cd* __restrict__ Tg = V + 3LL * n * HB;
-  cd* tau = tau_all + (long long)mat * n;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int r0 = i0 + 1;
-
-  for (int j = 0; j < nb; ++j) {
-    const int c = i0 + j;
-    const long long cc = (long long)c * n;
-    for (int r = r0 + tid; r < n; r += 256) sb[r] = A[r + cc];
-    // the reflector below reads sb with another row-to-thread mapping
-    __syncthreads();
-    if (j > 0) {
-      // b -= Y(:, 0:j) conj(V(c, 0:j))
-      if (tid < j) s_row[tid] = conj(V[c + (long long)tid * n]);
-      __syncthreads();
-      for (int r = r0 + tid; r < n; r += 256) {
-        cd acc = mk(0.0, 0.0);
-        for (int p = 0; p < j; ++p) acc += Y[r + (long long)p * n] * s_row[p];
-        sb[r] -= acc;
-      }
-      __syncthreads();
-      // b <- (I - V T^H V^H) b
-      for (int p = wave; p < j; p += 4) {
-        const cd* vp = V + (long long)p * n;
-        double ar = 0.0, ai = 0.0;
-        for (int r = r0 + lane; r < n; r += 64) {
-          const cd z = cmul(vp[r], sb[r]);
-          ar += z.re;
-          ai += z.im;
-        }
-        ar = wave_sum(ar);
-        ai = wave_sum(ai);
-        if (lane == 0) s_w[p] = mk(ar, ai);
-      }
-      __syncthreads();
-      if (tid < j) {
-        cd acc = mk(0.0, 0.0);
-        for (int q = 0; q <= tid; ++q) acc += conj(Ts[tid * (tid + 1) / 2 + q]) * s_w[q];
-        s_t[tid] = acc;
-      }
-      __syncthreads();
-      for (int r = r0 + tid; r < n; r += 256) {
-        cd acc = mk(0.0, 0.0);
-        for (int p = 0; p < j; ++p) acc += V[r + (long long)p * n] * s_t[p];
-        sb[r] -= acc;
-      }
-      __syncthreads();
-    }
-    // reflector of b(c+1 .. n-1) (zlarfg: H^H x = beta e1)
-    double part = 0.0;
-    for (int r = c + 2 + tid; r < n; r += 256) part += norm2(sb[r]);
-    const double xn2 = block_sum(part, sred);
-    if (tid == 0) {
-      const cd alpha = sb[c + 1];
-      cd beta = alpha;
-      if (xn2 == 0.0 && alpha.im == 0.0) {
-        s_tau = mk(0.0, 0.0);
-        s_scale = mk(0.0, 0.0);
-      } else {
-        const double nrm = sqrt(alpha.re * alpha.re + alpha.im * alpha.im + xn2);
-        const double bt = (alpha.re >= 0.0) ? -nrm : nrm;
-        s_tau = mk((bt - alpha.re) / bt, -alpha.im / bt);
-        s_scale = cinv(alpha - mk(bt, 0.0));
-        beta = mk(bt, 0.0);
-      }
-      tau[c] = s_tau;
-      sb[c + 1] = beta;
-    }
-    __syncthreads();
-    const cd t = s_tau, sc = s_scale;
-    cd* Vj = V + (long long)j * n;
-    for (int r = tid; r < n; r += 256) {
-      cd v = mk(0.0, 0.0);
-      if (r == c + 1) v = mk(1.0, 0.0);
-      else if (r > c + 1) v = sb[r] * sc;
-      sv[r] = v;
-      Vj[r] = v;
-      // column c of the reduced matrix: updated entries above the
-      // subdiagonal, beta on it, the reflector below it
-      if (r >= r0) A[r + cc] = (r > c + 1) ? v : sb[r];
-    }
-    __syncthreads();
-    // t = V(:, 0:j)^H v
-    for (int p = wave; p < j; p += 4) {
-      const cd* vp = V + (long long)p * n;
-      double ar = 0.0, ai = 0.0;
-      for (int r = c + 1 + lane; r < n; r += 64) {
-        const cd z = cmul(vp[r], sv[r]);
-        ar += z.re;
-        ai += z.im;
-      }
-      ar = wave_sum(ar);
-      ai = wave_sum(ai);
-      if (lane == 0) s_t[p] = mk(ar, ai);
-    }
-    __syncthreads();
-    // y = A(r0:n, c+1:n) v(c+1:n) over the block-start columns, then
-    // Y(:, j) = tau (y - Y(:, 0:j) t): two rows per thread, 512 rows a pass
-    for (int base = r0; base < n; base += 512) {
-      const int ra = base + tid, rb = base + tid + 256;
-      if (ra >= n) break;
-      const bool hb = rb < n;
-      cd ya = mk(0.0, 0.0), yb = mk(0.0, 0.0);
-#pragma unroll 4
-      for (int q = c + 1; q < n; ++q) {
-        const cd vq = sv[q];
-        const cd* col = A + (long long)q * n;
-        ya += col[ra] * vq;
-        if (hb) yb += col[rb] * vq;
-      }
-      cd acc = ya;
-      for (int p = 0; p < j; ++p) acc -= Y[ra + (long long)p * n] * s_t[p];
-      Y[ra + (long long)j * n] = t * acc;
-      if (hb) {
-        acc = yb;
-        for (int p = 0; p < j; ++p) acc -= Y[rb + (long long)p * n] * s_t[p];
-        Y[rb + (long long)j * n] = t * acc;
-      }
-    }
-    // T(0:j, j) = -tau T(0:j, 0:j) t,  T(j, j) = tau
-    if (tid < j) {
-      cd acc = mk(0.0, 0.0);
-      for (int q = tid; q < j; ++q) acc += Ts[q * (q + 1) / 2 + tid] * s_t[q];
-      Ts[j * (j + 1) / 2 + tid] = -(t * acc);
-    }
-    if (tid == j) Ts[j * (j + 1) / 2 + j] = t;
-    __syncthreads();
-  }
-  for (int e = tid; e < HB * HB; e += 256) {
-    const int r = e % HB, q = e / HB;
-    Tg[e] = (r <= q && q < nb) ? Ts[q * (q + 1) / 2 + r] : mk(0.0, 0.0);
-  }
-  // columns outside the panel of V stay zero for the GEMMs
-  for (long long e = (long long)nb * n + tid; e < (long long)HB * n; e += 256) V[e] = mk(0.0, 0.0);
-  if (tid == 0 && i0 + nb == n - 2) {
-    tau[n - 2] = mk(0.0, 0.0);
-    tau[n - 1] = mk(0.0, 0.0);
-  }
-}
-
 // The panel in two launches a column: k_hess_mv forms y = A v in
-// 64-row strips times nch column ranges per matrix (k_hess_panel, one workgroup
-// a matrix, streams it through one compute unit: 52 us a column at n = 450, 177
-// at n = 798), k_hess_col, one workgroup a matrix, finishes Y's column from the
+// 64-row strips times nch column ranges per matrix (one workgroup a matrix would
+// stream it through one compute unit: 52 us a column at n = 450, 177 at n = 798),
+// k_hess_col, one workgroup a matrix, finishes Y's column from the
 // partial sums (in the Ytmp region, free during the panel) and forms the next
 // reflector.  Launch order is the only synchronisation.  t and tau of the last
 // reflector wait in Z for the next call.
@@ -502,21 +346,13 @@ __global__ __launch_bounds__(256) void k_hess_mv(int n, int i0, int j, int cw, c
     P[r + (long long)blockIdx.y * n] = red[0][lane] + red[1][lane] + red[2][lane] + red[3][lane];
 }
 
-// Which panel kernel: the one workgroup a matrix only where matrices are small
-// and many.  Time of a pillar batch with the split panel / without, ms: n = 162,
-// 600 matrices 69.6 / 67.5; n = 242, 240: 74.5 / 74.8, 400: 91.9 / 93.5, 760:
-// 149 / 144; n = 450, 4: 121 / 136, 256: 235 / 262, 1280: 885 / 903; n = 722,
-// 3: 235 / 322.
-static bool hess_split(int n, int batch) { return n >= 300 || batch <= 512; }
-
-static void hess_panel_split(hipStream_t s, int n, int i0, int nb, cd* const* A, cd* tau,
-                           cd* const* X, cd* const* Z, int batch) {
+static void hess_panel(hipStream_t s, int n, int i0, int nb, cd* const* A, cd* tau,
+                       cd* const* X, cd* const* Z, int batch) {
   const int strips = (n - i0 - 1 + 63) / 64;
-  // column ranges: about 768 workgroups in all, at most 256 and at least 16
-  // columns each
-  int nch = std::min(768 / (strips * batch), (n - i0 - 1) / 16);
-  nch = std::min(std::max({nch, 1, (n - i0 - 1 + 255) / 256}), HB);
-  const int cw = (n - i0 - 1 + nch - 1) / nch;
+  // column ranges of a width that depends on n alone, so that a matrix's sums,
+  // and with them its eigenvalues' order, do not depend on what it is batched
+  // with; at least 32 columns, at most HB ranges
+  const int cw = std::max(64, (n + HB - 1) / HB), nch = (n - i0 - 2 + cw) / cw;
   for (int j = 0; j <= nb; ++j) {
     hipLaunchKernelGGL(k_hess_col, dim3(batch), dim3(HC_T), n * sizeof(cd), s, n, i0, j, nb, nch,
                        A, tau, X, Z);
@@ -536,11 +372,7 @@ static void hess_blocked(hipStream_t s, int n, cd* const* A, cd* tau, cd* const*
   for (int i0 = 0; i0 + 2 < n; i0 += HB) {
     const int nb = std::min(HB, n - 2 - i0);
     const int top = i0 + 1, m = n - i0 - 1, nt = n - i0 - nb;
-    if (hess_split(n, batch))
-      hess_panel_split(s, n, i0, nb, A, tau, X, Z, batch);
-    else
-      hipLaunchKernelGGL(k_hess_panel, dim3(batch), dim3(256), 2 * n * sizeof(cd), s, n, i0, nb,
-                         A, tau, X);
+    hess_panel(s, n, i0, nb, A, tau, X, Z, batch);
     // Ytmp(0:top) = A(0:top, i0+1:n) V(i0+1:n, :);  Y(0:top) = Ytmp T
     zgemm_batched(s, top, nb, m, one, Ac, (long long)top * n, 1, n, 0, Xc, oV + top, 1, n, 0,
                   zero, X, oYt, 1, n, batch);
@@ -864,12 +696,19 @@ __global__ void k_zero_counts(int* a, int n) {
   for (int i = threadIdx.x; i < n; i += blockDim.x) a[i] = 0;
 }
 
+// about twice what an RCWA matrix takes
+__host__ constexpr int qr_fixed_rounds(int n) { return 8 + n / 6; }
+
 // The rounds of the two-kernel form.  The host learns how many matrices are
 // left from a counter per round, read back only when about as many sweeps have
 // run as an RCWA matrix takes (n / 12), then every few rounds: a round that
-// finds nothing to do costs two empty launches.
+// finds nothing to do costs two empty launches.  Where the host may not wait (a
+// graph is captured) the rounds are qr_fixed_rounds(n), and the kernel of one workgroup
+// a matrix takes on whatever is left: the same iteration, so a replay agrees with
+// the eager solve.
 static void qr_rounds(hipStream_t s, int n, cd* const* A, cd* const* Z, cd* const* X,
-                      cd* const* W, int* counts, int ncounts, int* info, int batch) {
+                      cd* const* W, int* counts, int ncounts, int* info, int batch,
+                      bool host_wait) {
   const int maxsweep = 40 + 3 * n, strips = 3 * ((n + 63) / 64);
   const int nc = std::min(ncounts, 1024);
   int round = 0, check = std::max(2, n / 13);
@@ -880,7 +719,12 @@ static void qr_rounds(hipStream_t s, int n, cd* const* A, cd* const* Z, cd* cons
                        X, W, info, counts, maxsweep);
     hipLaunchKernelGGL(qr_w48::k_qr_apply, dim3(strips * batch), dim3(256), 0, s, n, batch, A, Z, X, W);
     ++round;
-    if (round < check) continue;
+    if (!host_wait && round == qr_fixed_rounds(n)) {
+      hipLaunchKernelGGL(qr_w48::k_qr_ms, dim3(batch), dim3(256), 0, s, n, A, Z,
+                         (const cd* const*)X, info, maxsweep);
+      return;
+    }
+    if (!host_wait || round < check) continue;
     check = round + 2;
     int left = 0;
     if (hipMemcpyAsync(&left, counts + slot, sizeof(int), hipMemcpyDeviceToHost, s) != hipSuccess ||
@@ -1156,20 +1000,21 @@ void zgeev_batched(hipStream_t s, int n, cd* const* A, const cd* const* Aorig, c
   if (ev) (void)hipEventRecord(ev[0], s);
   // zero everything below the first subdiagonal (the Householder vectors)
   hipLaunchKernelGGL(k_zero_below_subdiag, dim3(64, batch), dim3(256), 0, s, n, A);
-  if (host_wait && qr_variant == QR_W48 && qr_split(n, batch))
-    qr_rounds(s, n, A, ws.Z, ws.X, W, reinterpret_cast<int*>(ws.tau), 4 * n * batch, info, batch);
+  if (qr_variant == QR_W48 && qr_split(n, batch))
+    qr_rounds(s, n, A, ws.Z, ws.X, W, reinterpret_cast<int*>(ws.tau), 4 * n * batch, info, batch,
+              host_wait);
   else switch (qr_variant) {
     case QR_W32:
-      hipLaunchKernelGGL(qr_w32::k_qr_ms, dim3(batch), dim3(256), 0, s, n, A, ws.Z, info,
-                         40 + 3 * n);
+      hipLaunchKernelGGL(qr_w32::k_qr_ms, dim3(batch), dim3(256), 0, s, n, A, ws.Z, nullptr,
+                         info, 40 + 3 * n);
       break;
     case QR_W64:
-      hipLaunchKernelGGL(qr_w64::k_qr_ms, dim3(batch), dim3(256), 0, s, n, A, ws.Z, info,
-                         40 + 3 * n);
+      hipLaunchKernelGGL(qr_w64::k_qr_ms, dim3(batch), dim3(256), 0, s, n, A, ws.Z, nullptr,
+                         info, 40 + 3 * n);
       break;
     default:
-      hipLaunchKernelGGL(qr_w48::k_qr_ms, dim3(batch), dim3(256), 0, s, n, A, ws.Z, info,
-                         40 + 3 * n);
+      hipLaunchKernelGGL(qr_w48::k_qr_ms, dim3(batch), dim3(256), 0, s, n, A, ws.Z, nullptr,
+                         info, 40 + 3 * n);
   }
   if (ev) (void)hipEventRecord(ev[1], s);
   if (n >= 64)

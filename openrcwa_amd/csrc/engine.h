@@ -76,8 +76,8 @@ void copy_batched(hipStream_t s, long long count, const cd* const* A, cd* const*
 // (accepted when ||Aorig W - W diag(lam)||max / ||Aorig||max <= tol, else
 // ORCWA_STATUS_EIG_RESIDUAL); status bits are or-ed into info[b].  resid[b]
 // receives the relative residual.  host_wait: the launcher may wait for the
-// stream (the QR then runs in rounds until no matrix is left; not in a stream
-// capture).
+// stream (to see how many rounds of the QR are still needed); in a stream
+// capture it may not.
 struct EigWorkspace {
   cd** Z;        // [batch] n*n
   cd** X;        // [batch] n*n

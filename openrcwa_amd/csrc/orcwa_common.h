@@ -109,6 +109,17 @@ __device__ __forceinline__ void lds_st(cd* p, cd z) {
 }
 
 // wavefront (64-lane) helpers
+// value of a uniform lane, in scalar registers
+__device__ __forceinline__ double lane_value(double v, int lane) {
+  union { double d; int i[2]; } u;
+  u.d = v;
+  u.i[0] = __builtin_amdgcn_readlane(u.i[0], lane);
+  u.i[1] = __builtin_amdgcn_readlane(u.i[1], lane);
+  return u.d;
+}
+__device__ __forceinline__ cd lane_value(cd v, int lane) {
+  return mk(lane_value(v.re, lane), lane_value(v.im, lane));
+}
 __device__ inline double wave_sum(double v) {
   for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
   return v;
@@ -116,6 +127,19 @@ __device__ inline double wave_sum(double v) {
 __device__ inline double wave_max(double v) {
   for (int off = 32; off > 0; off >>= 1) v = fmax(v, __shfl_xor(v, off, 64));
   return v;
+}
+// q <- q with the interchanges k0 + j <-> (pivot in lane j), j < nb, applied in
+// order (q in LDS, on one wave: the pivots are in its lanes, so a step costs two
+// LDS latencies and no load from memory)
+__device__ __forceinline__ void compose_swaps(int k0, int nb, int pivot, int* q) {
+  for (int j = 0; j < nb; ++j) {
+    const int k = k0 + j, p = __builtin_amdgcn_readlane(pivot, j);
+    if (p != k) {
+      const int a = q[k], c = q[p];
+      q[k] = c;
+      q[p] = a;
+    }
+  }
 }
 // orders LDS accesses between the lanes of one wavefront
 __device__ inline void wave_fence() {

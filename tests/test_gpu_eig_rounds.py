@@ -29,3 +29,16 @@ def test_rounds_match_numpy(gpu_ctx, n, batch):
         d = np.abs(lam[b][:, None] - ref[None, :])
         assert d.min(1).max() <= tol and d.min(0).max() <= tol
         assert np.abs(np.linalg.norm(W[b], axis=0) - 1.0).max() <= 1e-12
+
+
+@pytest.mark.parametrize("n,batch", [(130, 40), (242, 9), (338, 16), (450, 27)])
+def test_same_matrix_in_any_batch(gpu_ctx, n, batch):
+    """A matrix's eigenvalues, their order included, do not depend on the batch it
+    is solved in (few matrices iterate in rounds, many in one kernel): a plan that
+    runs in chunks, or inside a captured graph, agrees with one that does not."""
+    rng = np.random.default_rng(n)
+    a = rng.normal(size=(batch, n, n)) + 1j * rng.normal(size=(batch, n, n))
+    lam, W, _, info = zgeev(gpu_ctx, a)
+    few = zgeev(gpu_ctx, a[:2])
+    assert not info.any() and not few[3].any()
+    assert np.array_equal(lam[:2], few[0]) and np.array_equal(W[:2], few[1])
