@@ -771,13 +771,6 @@ __device__ __forceinline__ double dpp_move(double v) {
   u.i[1] = __builtin_amdgcn_update_dpp(u.i[1], u.i[1], CTRL, 0xf, 0xf, false);
   return u.d;
 }
-__device__ __forceinline__ double lane_double(double v, int lane) {
-  union { double d; int i[2]; } u;
-  u.d = v;
-  u.i[0] = __builtin_amdgcn_readlane(u.i[0], lane);
-  u.i[1] = __builtin_amdgcn_readlane(u.i[1], lane);
-  return u.d;
-}
 // maximum over the first 16 lanes, and over the wave, in every lane (lanes
 // without a source keep their own)
 __device__ __forceinline__ double dpp_row_reduce(double v) {
@@ -787,13 +780,13 @@ __device__ __forceinline__ double dpp_row_reduce(double v) {
   return fmax(v, dpp_move<0x118>(v));   // row_shr:8
 }
 __device__ __forceinline__ double dpp_row_max(double v) {
-  return lane_double(dpp_row_reduce(v), 15);
+  return lane_value(dpp_row_reduce(v), 15);
 }
 __device__ __forceinline__ double dpp_wave_max(double v) {
   v = dpp_row_reduce(v);
   v = fmax(v, dpp_move<0x142>(v));   // row_bcast:15
   v = fmax(v, dpp_move<0x143>(v));   // row_bcast:31
-  return lane_double(v, 63);
+  return lane_value(v, 63);
 }
 
 // 1 / z: conj(z) times the Newton-refined reciprocal of |z|^2 (2 ulp; a tenth
@@ -977,28 +970,24 @@ __global__ __launch_bounds__(256) void k_laswp_panel(int n, int k0, int nb, cd* 
       if (s_src[t] != t) A[s_R[t]] = lds_ld(&tile[s_src[t]][c]);
 }
 
-// perm[r] = the original row that ends in row r after all n interchanges
-// (one thread per matrix, up to PERM_MB matrices per workgroup, in LDS)
-constexpr int PERM_MB = 16;
-__global__ __launch_bounds__(PERM_MB) void k_ipiv_to_perm(int n, const int* ipiv, int* perm,
-                                                          int batch) {
+// perm[r] = the original row that ends in row r after all n interchanges (one
+// wave per matrix, up to PERM_MB matrices per workgroup, in LDS)
+constexpr int PERM_MB = 4;
+__global__ __launch_bounds__(64 * PERM_MB) void k_ipiv_to_perm(int n, const int* ipiv, int* perm,
+                                                               int batch) {
   extern __shared__ int sp[];
-  const int b = blockIdx.x * blockDim.x + threadIdx.x;
-  int* q = sp + (long long)threadIdx.x * n;
-  if (b < batch) {
-    const int* pv = ipiv + (long long)b * n;
-    for (int r = 0; r < n; ++r) q[r] = r;
-    for (int k = 0; k < n; ++k) {
-      const int p = pv[k];
-      if (p != k) {
-        const int t = q[k];
-        q[k] = q[p];
-        q[p] = t;
-      }
-    }
-    int* out = perm + (long long)b * n;
-    for (int r = 0; r < n; ++r) out[r] = q[r];
-  }
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int b = blockIdx.x * (blockDim.x >> 6) + wave;
+  if (b >= batch) return;
+  int* q = sp + (long long)wave * n;
+  const int* pv = ipiv + (long long)b * n;
+  for (int r = lane; r < n; r += 64) q[r] = r;
+  wave_fence();
+  for (int k0 = 0; k0 < n; k0 += 64)
+    compose_swaps(k0, min(64, n - k0), k0 + lane < n ? pv[k0 + lane] : 0, q);
+  wave_fence();
+  int* out = perm + (long long)b * n;
+  for (int r = lane; r < n; r += 64) out[r] = q[r];
 }
 
 // B <- P^T B as a gather through LDS: ncw (<= PERM_NC) columns per workgroup
@@ -1167,7 +1156,7 @@ void zgetrs_batched(hipStream_t s, int n, int nrhs, const cd* const* LU, const i
   const int mb = (int)std::min<size_t>(PERM_MB, kPermLds / ((size_t)n * sizeof(int)));
   const int ncw = (int)std::min<size_t>(PERM_NC, kPermLds / ((size_t)n * sizeof(cd)));
   if (perm_ws && mb >= 1 && ncw >= 1) {
-    hipLaunchKernelGGL(k_ipiv_to_perm, dim3((batch + mb - 1) / mb), dim3(mb),
+    hipLaunchKernelGGL(k_ipiv_to_perm, dim3((batch + mb - 1) / mb), dim3(64 * mb),
                        (size_t)mb * n * sizeof(int), s, n, ipiv, perm_ws, batch);
     hipLaunchKernelGGL(k_apply_perm, dim3((nrhs + ncw - 1) / ncw, batch), dim3(256),
                        (size_t)ncw * n * sizeof(cd), s, n, nrhs, ncw, (const int*)perm_ws, B);

@@ -352,7 +352,8 @@ static int plan_create(orcwa_gpu_context* ctx, const orcwa_stack* st, const orcw
   if (!st->thickness) return fail("null thickness array");
   const int nx = 2 * st->nx_harm + 1, ny = 2 * st->ny_harm + 1;
   if (nx > 63 || ny > 63) return fail("at most 31 harmonics per axis are supported");
-  // the cascade's column chain holds 4 n-vectors in LDS (160 KB per workgroup)
+  // the cascade's column chain holds two n-vectors, the interchanges and its
+  // panels in LDS (160 KB per workgroup): 155 KB at this limit
   if (4 * (size_t)(2 * nx * ny) * sizeof(cd) > 160 * 1024)
     return fail("at most 1280 harmonics ((2Nx+1)(2Ny+1)) are supported");
   bool own_edges = (layer_cx != nullptr);
@@ -1398,8 +1399,8 @@ static int plan_run(orcwa_plan* p, hipStream_t s, bool graph) {
       const size_t tvb = 2 * (size_t)n * sizeof(cd);
       launch_cascade_tail(s, n, i0, p->dev<const cd* const*>(ct.LU[sl]),
                           p->d_spiv + (size_t)sl * p->chunk * n, C(E), C(H),
-                          sl > 0 ? p->dev<const cd* const*>(ct.Rt[sl & 1]) : nullptr, p->d_rtv,
-                          ni);
+                          sl > 0 ? p->dev<const cd* const*>(ct.Rt[sl & 1]) : nullptr,
+                          p->dev<cd* const*>(ct.Rt[(sl + 1) & 1]), p->d_rtv, ni);
       if (p->keep)
         HIPCHK(hipMemcpyAsync(p->d_tv + 2 * (size_t)n, p->d_rtv + 2 * (size_t)n, tvb,
                               hipMemcpyDeviceToDevice, s));

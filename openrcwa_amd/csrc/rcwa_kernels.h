@@ -133,9 +133,10 @@ void launch_pv_in(hipStream_t s, const ConvGeom& g, const ProbParam* params, con
                   cd* const* out, int batch);
 void launch_pv_out(hipStream_t s, const ConvGeom& g, const ProbParam* params, const cd* const* U,
                    long long offU, const cd* const* Vb, cd* const* H, int batch);
+// (U: an n x 2 scratch matrix an instance, used where Rt is given)
 void launch_cascade_tail(hipStream_t s, int n, int i0, const cd* const* LUt, const int* piv,
-                         const cd* const* A, const cd* const* B, const cd* const* Rt, cd* rt,
-                         int batch);
+                         const cd* const* A, const cd* const* B, const cd* const* Rt,
+                         cd* const* U, cd* rt, int batch);
 void launch_cascade_chain(hipStream_t s, int n, const cd* const* LUt, const int* piv,
                           const cd* const* keff, const double* k0d, cd* rt, int batch);
 void launch_field_combine(hipStream_t s, int n, int L, const cd* tv, cd px, cd py, cd* cp);

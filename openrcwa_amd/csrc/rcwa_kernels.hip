@@ -535,225 +535,292 @@ __global__ void k_pv_out(const ConvGeom g, const ProbParam* params, const cd* co
   }
 }
 
-// x <- M^-1 x for the two vectors x0, x1 (LDS), given zgetrf of M^T:
+// x <- M^-1 x for two vectors, given zgetrf of M^T:
 // M^T = P L U  =>  M = U^T L^T P^T  =>  x = P L^-T U^-T x.
-// Solved by the whole 256-thread workgroup, in blocks of TS rows:
-// per block the four waves first subtract the contributions of the entries
-// already solved (coalesced column reads of LU, one wave per row), then wave
-// 0 finishes the TS x TS triangle from LDS with one lane per row, each solved
-// entry broadcast by a lane shuffle.  2 n / TS barriers instead of a global
-// load latency per row.  Every thread of the workgroup must call it.
-constexpr int TS = 32;
-__device__ void lu_t_solve2(int n, const cd* __restrict__ LU,
-                            const int* __restrict__ piv, cd* x0, cd* x1,
-                            cd (*blk)[TS + 1]) {
+// One workgroup of LT_THREADS an instance, in blocks of TS rows; latency bounds
+// it (the n x n factors are read once, 32 us of 1 ms at n = 450), so the three
+// chains of a block run side by side on waves of their own and a block costs one
+// barrier:
+//  - wave 0 solves the TS x TS triangle, one lane a row, the solved entry
+//    broadcast through scalar registers; its upper 32 lanes meanwhile subtract
+//    the block from the TS rows that come next, so nobody waits for a correction.
+//    The rows of U come divided by their diagonal, which leaves eight fused
+//    operations a step;
+//  - waves 1 to 8 stage the next block's panel (TS x 2 TS) and subtract what the
+//    entries solved before this block give to its rows (four rows a wave, one
+//    read of x for all of them);
+//  - wave 9 composes the interchanges, TS a block, into q: afterwards z (in x0,
+//    x1) belongs at x[q[k]] = z[k].
+// One link of the chain at n = 450: 735 us with 256 threads, the three one after
+// the other and a thread that swapped for the interchanges; 232 us now.
+// Every thread of the workgroup must call it, after a barrier behind x0 and x1.
+constexpr int TS = 32, LT_THREADS = 640, LT_HELPERS = 8;
+constexpr int LT_PANEL = TS * (2 * TS + 1);   // panel[a][c]; panel[a][2 TS] = 1 / diagonal
+static_assert(LT_HELPERS * 4 == TS && (LT_HELPERS + 2) * 64 == LT_THREADS, "roles of the waves");
+__host__ __device__ constexpr size_t lt_lds(size_t n) {
+  return (2 * n + 2 * LT_PANEL) * sizeof(cd) + n * sizeof(int);
+}
+// sum_j col[j] x[j] for four columns of LU, j in [lo, hi); the lanes of a wave
+// share the range, lane l ends with component (l >> 2) & 15
+__device__ __forceinline__ double lt_dots(const cd* __restrict__ c0, const cd* __restrict__ c1,
+                                          const cd* __restrict__ c2, const cd* __restrict__ c3,
+                                          int lo, int hi, const cd* x0, const cd* x1, int lane) {
+  cd s[8];
+#pragma unroll
+  for (int k = 0; k < 8; ++k) s[k] = mk(0.0, 0.0);
+#pragma unroll 2
+  for (int j = lo + lane; j < hi; j += 64) {
+    const cd u0 = c0[j], u1 = c1[j], u2 = c2[j], u3 = c3[j];
+    const cd y0 = lds_ld(x0 + j), y1 = lds_ld(x1 + j);
+    s[0] = cfma(s[0], u0, y0);
+    s[1] = cfma(s[1], u0, y1);
+    s[2] = cfma(s[2], u1, y0);
+    s[3] = cfma(s[3], u1, y1);
+    s[4] = cfma(s[4], u2, y0);
+    s[5] = cfma(s[5], u2, y1);
+    s[6] = cfma(s[6], u3, y0);
+    s[7] = cfma(s[7], u3, y1);
+  }
+  // halving exchange: 8 + 4 + 2 + 1 sums instead of 16 x 4, then two full ones
+  double v[16];
+#pragma unroll
+  for (int k = 0; k < 8; ++k) {
+    v[2 * k] = s[k].re;
+    v[2 * k + 1] = s[k].im;
+  }
+#pragma unroll
+  for (int half = 8; half > 0; half >>= 1) {
+    const bool up = (lane & (4 * half)) != 0;
+#pragma unroll
+    for (int k = 0; k < half; ++k) {
+      const double keep = up ? v[k + half] : v[k], give = up ? v[k] : v[k + half];
+      v[k] = keep + __shfl_xor(give, 4 * half, 64);
+    }
+  }
+  v[0] += __shfl_xor(v[0], 2, 64);
+  return v[0] + __shfl_xor(v[0], 1, 64);
+}
+__device__ __forceinline__ void lu_t_solve2(int n, const cd* __restrict__ LU,
+                                            const int* __restrict__ piv, cd* x0, cd* x1,
+                                            cd* panel, int* q) {
   LU = gptr(LU);
+  piv = gptr(piv);
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int nblk = (n + TS - 1) / TS;
-  // U^T y = x, forward: y_i = (x_i - sum_{j<i} U(j,i) y_j) / U(i,i)
-  for (int bk = 0; bk < nblk; ++bk) {
-    const int r0 = bk * TS, nb = min(TS, n - r0);
-    for (int e = tid; e < nb * nb; e += 256) {
-      const int a = e % nb, c = e / nb;
-      blk[a][c] = LU[(r0 + a) + (long long)(r0 + c) * n];
+  const bool helper = wave >= 1 && wave <= LT_HELPERS;
+  // the panel of step t (forward: block t, backward: block 2 nblk - 1 - t); a
+  // helper's elements all lie in panel row a
+  const int ha = (tid - 64) & (TS - 1), hc = (tid - 64) >> 5;
+  cd pv[4], pd;
+  auto fetch = [&](int t) {
+    const bool fwd = t < nblk;
+    const int r0 = (fwd ? t : 2 * nblk - 1 - t) * TS, row = r0 + ha;
+    pd = mk(1.0, 0.0);
+    if (fwd && row < n) pd = LU[row + (long long)row * n];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int c = hc + 16 * i;
+      // columns of the block, then those of the rows that come next
+      const int col = (fwd || c < TS) ? r0 + c : r0 + c - 2 * TS;
+      const bool in = row < n && col >= 0 && col < n && (fwd ? c > ha : (c < ha || c >= TS));
+      pv[i] = mk(0.0, 0.0);
+      if (in) pv[i] = LU[row + (long long)col * n];
     }
-    for (int r = r0 + wave; r < r0 + nb; r += 4) {
-      const cd* col = LU + (long long)r * n;
-      double a0r = 0.0, a0i = 0.0, a1r = 0.0, a1i = 0.0;
-      for (int j = lane; j < r0; j += 64) {
-        const cd u = col[j], y0 = x0[j], y1 = x1[j];
-        a0r += u.re * y0.re - u.im * y0.im;
-        a0i += u.re * y0.im + u.im * y0.re;
-        a1r += u.re * y1.re - u.im * y1.im;
-        a1i += u.re * y1.im + u.im * y1.re;
-      }
-      a0r = wave_sum(a0r);
-      a0i = wave_sum(a0i);
-      a1r = wave_sum(a1r);
-      a1i = wave_sum(a1i);
-      if (lane == 0) {
-        x0[r] -= mk(a0r, a0i);
-        x1[r] -= mk(a1r, a1i);
-      }
-    }
-    __syncthreads();
-    if (wave == 0) {
-      cd v0 = mk(0.0, 0.0), v1 = mk(0.0, 0.0);
-      if (lane < nb) {
-        v0 = x0[r0 + lane];
-        v1 = x1[r0 + lane];
-      }
-      for (int k = 0; k < nb; ++k) {
-        if (lane == k) {
-          const cd d = cinv(blk[k][k]);
-          v0 = v0 * d;
-          v1 = v1 * d;
-        }
-        const cd y0 = mk(__shfl(v0.re, k, 64), __shfl(v0.im, k, 64));
-        const cd y1 = mk(__shfl(v1.re, k, 64), __shfl(v1.im, k, 64));
-        if (lane > k && lane < nb) {
-          const cd u = blk[k][lane];   // U(r0 + k, r0 + lane)
-          v0 -= u * y0;
-          v1 -= u * y1;
-        }
-      }
-      if (lane < nb) {
-        x0[r0 + lane] = v0;
-        x1[r0 + lane] = v1;
-      }
-    }
-    __syncthreads();
-  }
-  // L^T z = y, backward, unit diagonal: z_i = y_i - sum_{j>i} L(j,i) z_j
-  for (int bk = nblk - 1; bk >= 0; --bk) {
-    const int r0 = bk * TS, nb = min(TS, n - r0), r1 = r0 + nb;
-    for (int e = tid; e < nb * nb; e += 256) {
-      const int a = e % nb, c = e / nb;
-      blk[a][c] = LU[(r0 + a) + (long long)(r0 + c) * n];
-    }
-    for (int r = r0 + wave; r < r1; r += 4) {
-      const cd* col = LU + (long long)r * n;
-      double a0r = 0.0, a0i = 0.0, a1r = 0.0, a1i = 0.0;
-      for (int j = r1 + lane; j < n; j += 64) {
-        const cd l = col[j], z0 = x0[j], z1 = x1[j];
-        a0r += l.re * z0.re - l.im * z0.im;
-        a0i += l.re * z0.im + l.im * z0.re;
-        a1r += l.re * z1.re - l.im * z1.im;
-        a1i += l.re * z1.im + l.im * z1.re;
-      }
-      a0r = wave_sum(a0r);
-      a0i = wave_sum(a0i);
-      a1r = wave_sum(a1r);
-      a1i = wave_sum(a1i);
-      if (lane == 0) {
-        x0[r] -= mk(a0r, a0i);
-        x1[r] -= mk(a1r, a1i);
-      }
-    }
-    __syncthreads();
-    if (wave == 0) {
-      cd v0 = mk(0.0, 0.0), v1 = mk(0.0, 0.0);
-      if (lane < nb) {
-        v0 = x0[r0 + lane];
-        v1 = x1[r0 + lane];
-      }
-      for (int k = nb - 1; k >= 0; --k) {
-        const cd z0 = mk(__shfl(v0.re, k, 64), __shfl(v0.im, k, 64));
-        const cd z1 = mk(__shfl(v1.re, k, 64), __shfl(v1.im, k, 64));
-        if (lane < k) {
-          const cd l = blk[k][lane];   // L(r0 + k, r0 + lane)
-          v0 -= l * z0;
-          v1 -= l * z1;
-        }
-      }
-      if (lane < nb) {
-        x0[r0 + lane] = v0;
-        x1[r0 + lane] = v1;
-      }
-    }
-    __syncthreads();
-  }
-  // x = P z: the interchanges of zgetrf in reverse order
-  if (tid == 0) {
-    for (int k = n - 1; k >= 0; --k) {
-      const int p = piv[k];
-      if (p != k) {
-        cd t = x0[k]; x0[k] = x0[p]; x0[p] = t;
-        t = x1[k]; x1[k] = x1[p]; x1[p] = t;
-      }
-    }
+  };
+  auto stage = [&](int t) {
+    cd* p = panel + (t & 1) * LT_PANEL + ha * (2 * TS + 1);
+    const cd d = t < nblk ? cinv(pd) : mk(1.0, 0.0);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) lds_st(p + hc + 16 * i, t < nblk ? pv[i] * d : pv[i]);
+    if (hc == 0) lds_st(p + 2 * TS, d);
+  };
+  for (int i = tid; i < n; i += LT_THREADS) q[i] = i;
+  if (helper) {
+    fetch(0);
+    stage(0);
   }
   __syncthreads();
+  cd v0 = mk(0.0, 0.0), v1 = mk(0.0, 0.0);   // wave 0: the rows of its lanes
+  for (int t = 0; t < 2 * nblk; ++t) {
+    const bool fwd = t < nblk;
+    const int bk = fwd ? t : 2 * nblk - 1 - t;
+    const int r0 = bk * TS, nb = min(TS, n - r0);
+    if (wave == 0) {
+      const cd* p = panel + (t & 1) * LT_PANEL;
+      // what the block before left on these rows, from the upper lanes
+      const cd h0 = mk(__shfl_down(v0.re, 32, 64), __shfl_down(v0.im, 32, 64));
+      const cd h1 = mk(__shfl_down(v1.re, 32, 64), __shfl_down(v1.im, 32, 64));
+      v0 = v1 = mk(0.0, 0.0);
+      if (lane < nb) {
+        v0 = lds_ld(x0 + r0 + lane);
+        v1 = lds_ld(x1 + r0 + lane);
+        if (t != nblk) {
+          v0 += h0;
+          v1 += h1;
+        }
+      }
+      if (fwd) {
+#pragma unroll 8
+        for (int k = 0; k < TS; ++k) {
+          const cd y0 = lane_value(v0, k), y1 = lane_value(v1, k);
+          const cd u = lds_ld(p + k * (2 * TS + 1) + lane);   // 0 up to the diagonal
+          v0 = cfnma(v0, u, y0);
+          v1 = cfnma(v1, u, y1);
+        }
+      } else {
+#pragma unroll 8
+        for (int k = TS - 1; k >= 0; --k) {
+          const cd y0 = lane_value(v0, k), y1 = lane_value(v1, k);
+          const cd u = lds_ld(p + k * (2 * TS + 1) + lane);   // 0 from the diagonal on
+          v0 = cfnma(v0, u, y0);
+          v1 = cfnma(v1, u, y1);
+        }
+      }
+      if (lane < nb) {
+        const cd d = fwd ? lds_ld(p + lane * (2 * TS + 1) + 2 * TS) : mk(1.0, 0.0);
+        lds_st(x0 + r0 + lane, fwd ? v0 * d : v0);
+        lds_st(x1 + r0 + lane, fwd ? v1 * d : v1);
+      }
+    } else if (helper) {
+      if (t + 1 < 2 * nblk) {
+        fetch(t + 1);
+        // rows of the next block, against what was solved before this one
+        const int rn = fwd ? r0 + TS : r0 - TS;
+        const int lo = fwd ? 0 : r0 + nb, hi = fwd ? r0 : n;
+        if (t + 1 != nblk && lo < hi) {
+          const int r = rn + 4 * (wave - 1);
+          const cd* c = LU + (long long)min(r, n - 1) * n;
+          const cd* c1 = LU + (long long)min(r + 1, n - 1) * n;
+          const cd* c2 = LU + (long long)min(r + 2, n - 1) * n;
+          const cd* c3 = LU + (long long)min(r + 3, n - 1) * n;
+          const double sum = lt_dots(c, c1, c2, c3, lo, hi, x0, x1, lane);
+          const int comp = lane >> 2, rr = r + (comp >> 2);
+          if ((lane & 3) == 0 && rr < n) {
+            double* x = reinterpret_cast<double*>(((comp & 2) ? x1 : x0) + rr) + (comp & 1);
+            *x -= sum;
+          }
+        }
+        stage(t + 1);
+      }
+    } else if (fwd) {
+      compose_swaps(r0, nb, lane < nb ? piv[r0 + lane] : 0, q);
+    }
+    __syncthreads();
+  }
 }
 
 // Last cascade step (the interface at the incident half-space): for
 // c in {i0, h+i0}: x = (F+G)^-1 e_c, Rud e_c = (F-G) x = B x + A (R~ x),
 // 2 x starts the Tdd column chain.  Rt = R~^T of the previous steps, or null
-// for a two-layer stack.  One 256-thread workgroup per instance, LDS 4n cd.
-__global__ __launch_bounds__(256) void k_cascade_tail(int n, int i0, const cd* const* LUt,
-                                                      const int* piv_all, const cd* const* Ap,
-                                                      const cd* const* Bp, const cd* const* Rtp,
-                                                      cd* rt_all) {
-  extern __shared__ cd sm[];
+// for a two-layer stack.  The solve here, on one workgroup an instance; its
+// products with R~, A and B in the two kernels below, on the whole chip (in the
+// solve's workgroup they took 0.6 ms at n = 450).
+__global__ __launch_bounds__(LT_THREADS) void k_cascade_tail(int n, int i0,
+                                                             const cd* const* LUt,
+                                                             const int* piv_all, cd* rt_all) {
+  extern __shared__ __align__(16) cd sm[];
   cd* x0 = sm;
   cd* x1 = sm + n;
-  cd* u0 = sm + 2 * n;
-  cd* u1 = sm + 3 * n;
-  const int b = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  int* q = reinterpret_cast<int*>(sm + 2 * n + 2 * LT_PANEL);
+  const int b = blockIdx.x, tid = threadIdx.x;
   const int h = n / 2;
-  for (int i = tid; i < n; i += 256) {
+  for (int i = tid; i < n; i += LT_THREADS) {
     x0[i] = mk(i == i0 ? 1.0 : 0.0, 0.0);
     x1[i] = mk(i == h + i0 ? 1.0 : 0.0, 0.0);
   }
   __syncthreads();
-  // (the triangle blocks of the solve live where u0, u1 go afterwards)
-  lu_t_solve2(n, LUt[b], piv_all + (long long)b * n, x0, x1,
-              reinterpret_cast<cd(*)[TS + 1]>(u0));
-  // u = R~ x, R~(i, j) = Rt(j, i): column i of Rt
-  const cd* Rt = Rtp ? gptr(Rtp[b]) : nullptr;
-  for (int i = wave; i < n; i += 4) {
-    double a0r = 0.0, a0i = 0.0, a1r = 0.0, a1i = 0.0;
-    if (Rt) {
-      const cd* col = Rt + (long long)i * n;
-      for (int j = lane; j < n; j += 64) {
-        const cd r = col[j], y0 = x0[j], y1 = x1[j];
-        a0r += r.re * y0.re - r.im * y0.im;
-        a0i += r.re * y0.im + r.im * y0.re;
-        a1r += r.re * y1.re - r.im * y1.im;
-        a1i += r.re * y1.im + r.im * y1.re;
-      }
-      a0r = wave_sum(a0r);
-      a0i = wave_sum(a0i);
-      a1r = wave_sum(a1r);
-      a1i = wave_sum(a1i);
-    }
-    if (lane == 0) {
-      u0[i] = mk(a0r, a0i);
-      u1[i] = mk(a1r, a1i);
+  lu_t_solve2(n, LUt[b], piv_all + (long long)b * n, x0, x1, sm + 2 * n, q);
+  cd* out = rt_all + (long long)b * 4 * n;
+  for (int i = tid; i < n; i += LT_THREADS) {
+    out[2 * n + q[i]] = 2.0 * x0[i];
+    out[3 * n + q[i]] = 2.0 * x1[i];
+  }
+}
+
+// U[c][i] = 2 (R~ x_c)_i, R~(i, j) = Rt(j, i), from the 2 x in the chain's
+// columns; one wave an i
+__global__ __launch_bounds__(256) void k_cascade_rx(int n, const cd* const* Rtp,
+                                                    const cd* rt_all, cd* const* Up) {
+  const int b = blockIdx.y, lane = threadIdx.x & 63, i = blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (i >= n) return;
+  const cd* col = gptr(Rtp[b]) + (long long)i * n;
+  const cd* x = rt_all + (long long)b * 4 * n + 2 * n;
+  cd s0 = mk(0.0, 0.0), s1 = mk(0.0, 0.0);
+  for (int j = lane; j < n; j += 64) {
+    const cd r = col[j];
+    s0 = cfma(s0, r, x[j]);
+    s1 = cfma(s1, r, x[n + j]);
+  }
+  s0 = mk(wave_sum(s0.re), wave_sum(s0.im));
+  s1 = mk(wave_sum(s1.re), wave_sum(s1.im));
+  if (lane == 0) {
+    cd* U = gptr(Up[b]);
+    U[i] = s0;
+    U[n + i] = s1;
+  }
+}
+
+// The Rud columns from 2 x and U: 64 rows a workgroup, one lane a row, the
+// columns of A and B dealt to its 16 waves
+constexpr int CR_WAVES = 16;
+__global__ __launch_bounds__(64 * CR_WAVES) void k_cascade_rud(int n, const cd* const* Ap,
+                                                               const cd* const* Bp,
+                                                               const cd* const* Up, cd* rt_all) {
+  __shared__ alignas(16) cd part[CR_WAVES][2][64];
+  const int b = blockIdx.y, lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int i = blockIdx.x * 64 + lane, row = min(i, n - 1);
+  const cd* A = gptr(Ap[b]) + row;
+  const cd* B = gptr(Bp[b]) + row;
+  const cd* U = Up ? gptr(Up[b]) : nullptr;
+  cd* out = rt_all + (long long)b * 4 * n;
+  const cd* x = out + 2 * n;
+  cd r0 = mk(0.0, 0.0), r1 = mk(0.0, 0.0);
+  for (int j = wave; j < n; j += CR_WAVES) {
+    const cd bij = B[(long long)j * n];
+    r0 = cfma(r0, bij, x[j]);
+    r1 = cfma(r1, bij, x[n + j]);
+    if (U) {
+      const cd aij = A[(long long)j * n];
+      r0 = cfma(r0, aij, U[j]);
+      r1 = cfma(r1, aij, U[n + j]);
     }
   }
+  lds_st(&part[wave][0][lane], r0);
+  lds_st(&part[wave][1][lane], r1);
   __syncthreads();
-  const cd* A = gptr(Ap[b]);
-  const cd* B = gptr(Bp[b]);
-  cd* out = rt_all + (long long)b * 4 * n;
-  for (int i = tid; i < n; i += 256) {
-    cd r0 = mk(0.0, 0.0), r1 = mk(0.0, 0.0);
-    for (int j = 0; j < n; ++j) {
-      const cd bij = B[i + (long long)j * n], aij = A[i + (long long)j * n];
-      r0 += bij * x0[j] + aij * u0[j];
-      r1 += bij * x1[j] + aij * u1[j];
-    }
-    out[i] = r0;
-    out[n + i] = r1;
-    out[2 * n + i] = 2.0 * x0[i];
-    out[3 * n + i] = 2.0 * x1[i];
+  if (wave < 2 && i < n) {
+    cd r = mk(0.0, 0.0);
+    for (int w = 0; w < CR_WAVES; ++w) r += lds_ld(&part[w][wave][lane]);
+    out[wave * n + i] = 0.5 * r;
   }
 }
 
 // One link of the Tdd column chain: t <- 2 (F+G)_s^-1 (phi_{s+1} t), with
 // phi = exp(i keff (k0 d)) of the layer propagated at step s+1.
-__global__ __launch_bounds__(256) void k_cascade_chain(int n, const cd* const* LUt,
-                                                       const int* piv_all, const cd* const* keff,
-                                                       const double* k0d, cd* rt_all) {
-  extern __shared__ cd sm[];
-  __shared__ cd blk[TS][TS + 1];
+__global__ __launch_bounds__(LT_THREADS) void k_cascade_chain(int n, const cd* const* LUt,
+                                                              const int* piv_all,
+                                                              const cd* const* keff,
+                                                              const double* k0d, cd* rt_all) {
+  extern __shared__ __align__(16) cd sm[];
   cd* x0 = sm;
   cd* x1 = sm + n;
+  int* q = reinterpret_cast<int*>(sm + 2 * n + 2 * LT_PANEL);
   const int b = blockIdx.x, tid = threadIdx.x;
   cd* t = rt_all + (long long)b * 4 * n + 2 * n;
   const cd* kf = gptr(keff[b]);
   const double kd = k0d[b];
-  for (int i = tid; i < n; i += 256) {
+  for (int i = tid; i < n; i += LT_THREADS) {
     const cd a = kd * kf[i];
     const cd ph = cexp(mk(-a.im, a.re));
     x0[i] = t[i] * ph;
     x1[i] = t[n + i] * ph;
   }
   __syncthreads();
-  lu_t_solve2(n, LUt[b], piv_all + (long long)b * n, x0, x1, blk);
-  for (int i = tid; i < n; i += 256) {
-    t[i] = 2.0 * x0[i];
-    t[n + i] = 2.0 * x1[i];
+  lu_t_solve2(n, LUt[b], piv_all + (long long)b * n, x0, x1, sm + 2 * n, q);
+  for (int i = tid; i < n; i += LT_THREADS) {
+    t[q[i]] = 2.0 * x0[i];
+    t[n + q[i]] = 2.0 * x1[i];
   }
 }
 
@@ -967,19 +1034,22 @@ void launch_pv_out(hipStream_t s, const ConvGeom& g, const ProbParam* params, co
 }
 
 void launch_cascade_tail(hipStream_t s, int n, int i0, const cd* const* LUt, const int* piv,
-                         const cd* const* A, const cd* const* B, const cd* const* Rt, cd* rt,
-                         int batch) {
+                         const cd* const* A, const cd* const* B, const cd* const* Rt,
+                         cd* const* U, cd* rt, int batch) {
   if (batch <= 0) return;
-  // x0, x1, u0, u1; u0 onwards also holds the TS x (TS + 1) blocks of the solve
-  const size_t lds = (size_t)std::max(4 * n, 2 * n + TS * (TS + 1)) * sizeof(cd);
-  hipLaunchKernelGGL(k_cascade_tail, dim3(batch), dim3(256), lds, s, n, i0, LUt, piv, A, B, Rt,
+  hipLaunchKernelGGL(k_cascade_tail, dim3(batch), dim3(LT_THREADS), lt_lds(n), s, n, i0, LUt, piv,
                      rt);
+  if (Rt)
+    hipLaunchKernelGGL(k_cascade_rx, dim3((n + 3) / 4, batch), dim3(256), 0, s, n, Rt,
+                       (const cd*)rt, U);
+  hipLaunchKernelGGL(k_cascade_rud, dim3((n + 63) / 64, batch), dim3(64 * CR_WAVES), 0, s, n, A, B,
+                     Rt ? (const cd* const*)U : nullptr, rt);
 }
 
 void launch_cascade_chain(hipStream_t s, int n, const cd* const* LUt, const int* piv,
                           const cd* const* keff, const double* k0d, cd* rt, int batch) {
   if (batch <= 0) return;
-  hipLaunchKernelGGL(k_cascade_chain, dim3(batch), dim3(256), 2 * n * sizeof(cd), s, n, LUt, piv,
+  hipLaunchKernelGGL(k_cascade_chain, dim3(batch), dim3(LT_THREADS), lt_lds(n), s, n, LUt, piv,
                      keff, k0d, rt);
 }
 
