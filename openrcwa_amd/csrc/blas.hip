@@ -762,31 +762,9 @@ struct GetrfRegState {
   const int* info_map;
 };
 
-// value of lane (lane + shift inside the row / row broadcasts) of a double
-template <int CTRL>
-__device__ __forceinline__ double dpp_move(double v) {
-  union { double d; int i[2]; } u;
-  u.d = v;
-  u.i[0] = __builtin_amdgcn_update_dpp(u.i[0], u.i[0], CTRL, 0xf, 0xf, false);
-  u.i[1] = __builtin_amdgcn_update_dpp(u.i[1], u.i[1], CTRL, 0xf, 0xf, false);
-  return u.d;
-}
-// maximum over the first 16 lanes, and over the wave, in every lane (lanes
-// without a source keep their own)
-__device__ __forceinline__ double dpp_row_reduce(double v) {
-  v = fmax(v, dpp_move<0x111>(v));   // row_shr:1
-  v = fmax(v, dpp_move<0x112>(v));   // row_shr:2
-  v = fmax(v, dpp_move<0x114>(v));   // row_shr:4
-  return fmax(v, dpp_move<0x118>(v));   // row_shr:8
-}
+// maximum over the first 16 lanes, in every lane
 __device__ __forceinline__ double dpp_row_max(double v) {
-  return lane_value(dpp_row_reduce(v), 15);
-}
-__device__ __forceinline__ double dpp_wave_max(double v) {
-  v = dpp_row_reduce(v);
-  v = fmax(v, dpp_move<0x142>(v));   // row_bcast:15
-  v = fmax(v, dpp_move<0x143>(v));   // row_bcast:31
-  return lane_value(v, 63);
+  return lane_value(dpp_row_reduce_max(v), 15);
 }
 
 // 1 / z: conj(z) times the Newton-refined reciprocal of |z|^2 (2 ulp; a tenth
@@ -813,7 +791,7 @@ __device__ __forceinline__ void getrf_reg_step(GetrfRegState<T, WB>& S, cd (&a)[
       const bool in = S.pos >= c && S.pos < S.n;
       const double v0 = cabs1(a[J]);
       const double v = in ? (v0 == v0 ? v0 : 0.0) : -1.0;
-      const double best = dpp_wave_max(v);
+      const double best = wave_max(v);
       if (best >= 0.0) {
         unsigned long long who = __ballot(v == best);
         int bl = __ffsll(who) - 1, bp = __builtin_amdgcn_readlane(S.pos, bl);

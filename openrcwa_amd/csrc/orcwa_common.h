@@ -120,13 +120,39 @@ __device__ __forceinline__ double lane_value(double v, int lane) {
 __device__ __forceinline__ cd lane_value(cd v, int lane) {
   return mk(lane_value(v.re, lane), lane_value(v.im, lane));
 }
-__device__ inline double wave_sum(double v) {
-  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-  return v;
+// sum and maximum over the wave, in every lane (all lanes active): six moves
+// within the vector unit; as lane shuffles through LDS a sum took about five
+// times as long, and the serial kernels are made of such sums
+template <int CTRL, int ROWS>
+__device__ __forceinline__ double dpp_move(double old, double v) {
+  union { double d; int i[2]; } u, o;
+  u.d = v;
+  o.d = old;
+  u.i[0] = __builtin_amdgcn_update_dpp(o.i[0], u.i[0], CTRL, ROWS, 0xf, false);
+  u.i[1] = __builtin_amdgcn_update_dpp(o.i[1], u.i[1], CTRL, ROWS, 0xf, false);
+  return u.d;
 }
-__device__ inline double wave_max(double v) {
-  for (int off = 32; off > 0; off >>= 1) v = fmax(v, __shfl_xor(v, off, 64));
-  return v;
+__device__ __forceinline__ double wave_sum(double v) {
+  v += dpp_move<0x111, 0xf>(0.0, v);   // row_shr:1 (lanes without a source take 0)
+  v += dpp_move<0x112, 0xf>(0.0, v);   // row_shr:2
+  v += dpp_move<0x114, 0xf>(0.0, v);   // row_shr:4
+  v += dpp_move<0x118, 0xf>(0.0, v);   // row_shr:8
+  v += dpp_move<0x142, 0xa>(0.0, v);   // row_bcast:15 into rows 1 and 3
+  v += dpp_move<0x143, 0xc>(0.0, v);   // row_bcast:31 into rows 2 and 3
+  return lane_value(v, 63);
+}
+// maximum over the first 16 lanes in lane 15 (lanes without a source keep theirs)
+__device__ __forceinline__ double dpp_row_reduce_max(double v) {
+  v = fmax(v, dpp_move<0x111, 0xf>(v, v));
+  v = fmax(v, dpp_move<0x112, 0xf>(v, v));
+  v = fmax(v, dpp_move<0x114, 0xf>(v, v));
+  return fmax(v, dpp_move<0x118, 0xf>(v, v));
+}
+__device__ __forceinline__ double wave_max(double v) {
+  v = dpp_row_reduce_max(v);
+  v = fmax(v, dpp_move<0x142, 0xf>(v, v));
+  v = fmax(v, dpp_move<0x143, 0xf>(v, v));
+  return lane_value(v, 63);
 }
 // q <- q with the interchanges k0 + j <-> (pivot in lane j), j < nb, applied in
 // order (q in LDS, on one wave: the pivots are in its lanes, so a step costs two
