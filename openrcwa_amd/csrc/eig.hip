@@ -167,7 +167,29 @@ constexpr int HB = 32;
 // partial sums (in the Ytmp region, free during the panel) and forms the next
 // reflector.  Launch order is the only synchronisation.  t and tau of the last
 // reflector wait in Z for the next call.
-constexpr int HC_T = 512;
+constexpr int HC_T = 512, HC_W = HC_T / 64;
+// out[p] = V(lo:n, p)^H b for p < j: two columns a wave at a time
+__device__ __forceinline__ void hess_dots(const cd* V, int n, int lo, int j, const cd* sb, cd* out,
+                                          int wave, int lane) {
+  for (int p = wave; p < j; p += 2 * HC_W) {
+    const bool two = p + HC_W < j;
+    const cd* vp = V + (long long)p * n;
+    const cd* vq = two ? vp + (long long)HC_W * n : vp;
+    cd a = mk(0.0, 0.0), b = mk(0.0, 0.0);
+#pragma unroll 4
+    for (int r = lo + lane; r < n; r += 64) {
+      const cd s = sb[r];
+      a = cfmac(a, vp[r], s);
+      b = cfmac(b, vq[r], s);
+    }
+    a = mk(wave_sum(a.re), wave_sum(a.im));
+    b = mk(wave_sum(b.re), wave_sum(b.im));
+    if (lane == 0) {
+      out[p] = a;
+      if (two) out[p + HC_W] = b;
+    }
+  }
+}
 __global__ __launch_bounds__(HC_T) void k_hess_col(int n, int i0, int j, int nb, int nch,
                                                    cd* const* Ap, cd* tau_all, cd* const* Xp,
                                                    cd* const* Zp) {
@@ -210,15 +232,15 @@ __global__ __launch_bounds__(HC_T) void k_hess_col(int n, int i0, int j, int nb,
     if (j > 0) {
       cd y = mk(0.0, 0.0);
       for (int q = 0; q < nch; ++q) y += P[r + (long long)q * n];
-#pragma unroll 4
+#pragma unroll 8
       for (int p = 0; p + 1 < j; ++p) {
         const cd yp = Y[r + (long long)p * n];
-        y -= yp * s_told[p];
-        b -= yp * s_row[p];
+        y = cfnma(y, yp, s_told[p]);
+        b = cfnma(b, yp, s_row[p]);
       }
       y = told * y;
       Y[r + (long long)(j - 1) * n] = y;
-      b -= y * s_row[j - 1];
+      b = cfnma(b, y, s_row[j - 1]);
     }
     sb[r] = b;
   }
@@ -232,30 +254,22 @@ __global__ __launch_bounds__(HC_T) void k_hess_col(int n, int i0, int j, int nb,
   __syncthreads();
   if (j > 0) {
     // b <- (I - V T^H V^H) b
-    for (int p = wave; p < j; p += HC_T / 64) {
-      const cd* vp = V + (long long)p * n;
-      double ar = 0.0, ai = 0.0;
-#pragma unroll 4
-      for (int r = r0 + lane; r < n; r += 64) {
-        const cd z = cmul(vp[r], sb[r]);
-        ar += z.re;
-        ai += z.im;
-      }
-      ar = wave_sum(ar);
-      ai = wave_sum(ai);
-      if (lane == 0) s_w[p] = mk(ar, ai);
-    }
+    hess_dots(V, n, r0, j, sb, s_w, wave, lane);
     __syncthreads();
     if (tid < j) {
       cd acc = mk(0.0, 0.0);
-      for (int q = 0; q <= tid; ++q) acc += conj(Ts[tid * (tid + 1) / 2 + q]) * s_w[q];
+#pragma unroll 4
+      for (int q = 0; q < j; ++q) {     // (past the diagonal: reads T's next columns)
+        const cd u = Ts[tid * (tid + 1) / 2 + q], w = s_w[q];
+        if (q <= tid) acc = cfmac(acc, u, w);
+      }
       s_t[tid] = acc;
     }
     __syncthreads();
     for (int r = r0 + tid; r < n; r += HC_T) {
       cd acc = mk(0.0, 0.0);
-#pragma unroll 4
-      for (int p = 0; p < j; ++p) acc += V[r + (long long)p * n] * s_t[p];
+#pragma unroll 8
+      for (int p = 0; p < j; ++p) acc = cfma(acc, V[r + (long long)p * n], s_t[p]);
       sb[r] -= acc;
     }
     __syncthreads();
@@ -299,24 +313,16 @@ __global__ __launch_bounds__(HC_T) void k_hess_col(int n, int i0, int j, int nb,
   }
   __syncthreads();
   // t = V(:, 0:j)^H v
-  for (int p = wave; p < j; p += HC_T / 64) {
-    const cd* vp = V + (long long)p * n;
-    double ar = 0.0, ai = 0.0;
-#pragma unroll 4
-    for (int r = c + 1 + lane; r < n; r += 64) {
-      const cd z = cmul(vp[r], sb[r]);
-      ar += z.re;
-      ai += z.im;
-    }
-    ar = wave_sum(ar);
-    ai = wave_sum(ai);
-    if (lane == 0) s_t[p] = mk(ar, ai);
-  }
+  hess_dots(V, n, c + 1, j, sb, s_t, wave, lane);
   __syncthreads();
   // T(0:j, j) = -tau T(0:j, 0:j) t,  T(j, j) = tau
   if (tid < j) {
     cd acc = mk(0.0, 0.0);
-    for (int q = tid; q < j; ++q) acc += Ts[q * (q + 1) / 2 + tid] * s_t[q];
+#pragma unroll 4
+    for (int q = 0; q < j; ++q) {
+      const cd u = Ts[q * (q + 1) / 2 + min(tid, q)], w = s_t[q];
+      if (q >= tid) acc = cfma(acc, u, w);
+    }
     Tg[tid + j * HB] = -(t * acc);
     tz[tid] = s_t[tid];
   }
@@ -835,15 +841,18 @@ static void trevc_blocked(hipStream_t s, int n, const cd* const* T, cd* const* X
   }
 }
 
-// lam[j] = T[j,j]; unit 2-norm columns of W; relative residual.
+// lam[j] = T[j,j]; unit 2-norm columns of W: EF_COLS columns per workgroup (one
+// workgroup a matrix took 0.47 ms at n = 450, this 0.02).
+constexpr int EF_COLS = 16;
 __global__ __launch_bounds__(256) void k_eig_finish(int n, const cd* const* Tp, cd* const* Wp,
                                                     cd* lam) {
-  const int b = blockIdx.x;
+  const int b = blockIdx.y;
+  const int j0 = blockIdx.x * EF_COLS, j1 = min(n, j0 + EF_COLS);
   const cd* T = gptr(Tp[b]);
   cd* W = gptr(Wp[b]);
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  for (int j = tid; j < n; j += 256) lam[(long long)b * n + j] = T[j + (long long)j * n];
-  for (int j = wave; j < n; j += 4) {
+  if (j0 + tid < j1) lam[(long long)b * n + j0 + tid] = T[(j0 + tid) + (long long)(j0 + tid) * n];
+  for (int j = j0 + wave; j < j1; j += 4) {
     cd* col = W + (long long)j * n;
     double s = 0.0;
     for (int i = lane; i < n; i += 64) s += norm2(col[i]);
@@ -854,39 +863,50 @@ __global__ __launch_bounds__(256) void k_eig_finish(int n, const cd* const* Tp, 
 }
 
 // R = A W already in Rp; residual = max|R - W diag(lam)| / max|A|, accepted
-// when <= tol (1e-8 in the reference, rcwa/MKLEigenSolver.hpp:75-79)
+// when <= tol (1e-8 in the reference, rcwa/MKLEigenSolver.hpp:75-79).  The
+// maxima of strips of EF_COLS columns go to part ([matrix][strip][2]), a second
+// launch combines them (one workgroup a matrix took 0.45 ms at n = 450).
 __global__ __launch_bounds__(256) void k_eig_residual(int n, const cd* const* Ap,
                                                       const cd* const* Wp, const cd* const* Rp,
-                                                      const cd* lam, double* resid, int* info,
-                                                      double tol) {
-  __shared__ double sred[4];
-  const int b = blockIdx.x;
-  const cd* A = gptr(Ap[b]);
-  const cd* W = gptr(Wp[b]);
-  const cd* R = gptr(Rp[b]);
+                                                      const cd* lam, double* part) {
+  __shared__ double sr[4], sa[4];
+  const int b = blockIdx.y;
+  const int j0 = blockIdx.x * EF_COLS, j1 = min(n, j0 + EF_COLS);
+  const cd* A = gptr(Ap[b]) + (long long)j0 * n;
+  const cd* W = gptr(Wp[b]) + (long long)j0 * n;
+  const cd* R = gptr(Rp[b]) + (long long)j0 * n;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const long long nn = (long long)n * n;
   double ma = 0.0, mr = 0.0;
-  for (long long e = tid; e < nn; e += 256) {
+  for (int e = tid; e < (j1 - j0) * n; e += 256) {
     ma = fmax(ma, cabs(A[e]));
-    const cd l = lam[(long long)b * n + e / n];
+    const cd l = lam[(long long)b * n + j0 + e / n];
     mr = fmax(mr, cabs(R[e] - W[e] * l));
   }
   ma = wave_max(ma);
   mr = wave_max(mr);
-  __shared__ double sa[4];
   if (lane == 0) {
     sa[wave] = ma;
-    sred[wave] = mr;
+    sr[wave] = mr;
   }
   __syncthreads();
   if (tid == 0) {
-    const double a = fmax(fmax(sa[0], sa[1]), fmax(sa[2], sa[3]));
-    const double r = fmax(fmax(sred[0], sred[1]), fmax(sred[2], sred[3]));
-    const double rel = (a > 0.0) ? r / a : 0.0;
-    resid[b] = rel;
-    if (!(rel <= tol)) info[b] |= ORCWA_STATUS_EIG_RESIDUAL;
+    double* o = part + 2 * ((long long)b * gridDim.x + blockIdx.x);
+    o[0] = fmax(fmax(sa[0], sa[1]), fmax(sa[2], sa[3]));
+    o[1] = fmax(fmax(sr[0], sr[1]), fmax(sr[2], sr[3]));
   }
+}
+__global__ void k_eig_residual_max(int strips, const double* part, double* resid, int* info,
+                                   double tol, int batch) {
+  const int b = blockIdx.x * blockDim.x + threadIdx.x;
+  if (b >= batch) return;
+  double a = 0.0, r = 0.0;
+  for (int k = 0; k < strips; ++k) {
+    a = fmax(a, part[2 * ((long long)b * strips + k)]);
+    r = fmax(r, part[2 * ((long long)b * strips + k) + 1]);
+  }
+  const double rel = (a > 0.0) ? r / a : 0.0;
+  resid[b] = rel;
+  if (!(rel <= tol)) info[b] |= ORCWA_STATUS_EIG_RESIDUAL;
 }
 
 __global__ void k_zero_below_subdiag(int n, cd* const* Ap) {
@@ -1024,13 +1044,18 @@ void zgeev_batched(hipStream_t s, int n, cd* const* A, const cd* const* Aorig, c
   // W = Z X, X upper triangular (the eigenvectors of T)
   zgemm_batched_upper_b(s, n, n, n, mk(1.0, 0.0), (const cd* const*)ws.Z, 0, 1, n, 0,
                         (const cd* const*)ws.X, 0, 1, n, 0, mk(0.0, 0.0), W, 0, 1, n, batch);
-  hipLaunchKernelGGL(k_eig_finish, dim3(batch), dim3(256), 0, s, n, Ac, W, lam);
+  hipLaunchKernelGGL(k_eig_finish, dim3((n + EF_COLS - 1) / EF_COLS, batch), dim3(256), 0, s, n,
+                     Ac, W, lam);
   if (Aorig) {
     zgemm_batched(s, n, n, n, mk(1.0, 0.0), Aorig, 0, 1, n, 0, (const cd* const*)W, 0, 1, n, 0,
                   mk(0.0, 0.0), scratch, 0, 1, n, batch);
-    hipLaunchKernelGGL(k_eig_residual, dim3(batch), dim3(256), 0, s, n, Aorig,
-                       (const cd* const*)W, (const cd* const*)scratch, (const cd*)lam, resid,
-                       info, tol);
+    // (tau has been used up: the strips' maxima go there)
+    const int strips = (n + EF_COLS - 1) / EF_COLS;
+    double* part = reinterpret_cast<double*>(ws.tau);
+    hipLaunchKernelGGL(k_eig_residual, dim3(strips, batch), dim3(256), 0, s, n, Aorig,
+                       (const cd* const*)W, (const cd* const*)scratch, (const cd*)lam, part);
+    hipLaunchKernelGGL(k_eig_residual_max, dim3((batch + 63) / 64), dim3(64), 0, s, strips, part,
+                       resid, info, tol, batch);
   }
   if (ev) (void)hipEventRecord(ev[2], s);
 }
