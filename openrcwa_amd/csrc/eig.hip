@@ -583,12 +583,14 @@ __device__ __forceinline__ double rcp_shift(double v) {
   return fma(y, fma(-v, y, 1.0), y);
 }
 
-// the rotation, where neither norm is near the ends of the range (false otherwise)
+// the rotation, where neither norm is near the ends of the range (false otherwise);
+// the fusions are fixed, so that every kernel gets the same bits
 __device__ __forceinline__ bool rot_gen_fast(cd x0, cd x1, Rot& g) {
-  const double n0 = norm2(x0), n = n0 + norm2(x1);
+  const double n0 = fma(x0.re, x0.re, x0.im * x0.im);
+  const double n = n0 + fma(x1.re, x1.re, x1.im * x1.im);
   const double t = rsqrt_n(n0) * rsqrt_n(n);
   g.c = n0 * t;
-  g.s = t * mulc(x1, x0);
+  g.s = t * mk(fma(x1.re, x0.re, x1.im * x0.im), fma(x1.im, x0.re, -(x1.re * x0.im)));
   g.r = (n * t) * x0;
   return n0 > 1e-280 && n < 1e280;
 }
