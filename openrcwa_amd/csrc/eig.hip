@@ -652,14 +652,16 @@ __host__ __device__ constexpr int qr_slots(int n) {
 // rows apart, but for a few at the ends).  A round lasts as long as its slowest
 // matrix, so the more matrices there are, the more is lost against one
 // workgroup a matrix running through; the larger n is, the more the applies
-// gain.  One pillar stack of 4 layers, ms in rounds / in one kernel: n = 242
-// with 4 matrices 57.8 / 58.1, 32: 66 / 60; n = 338, 4: 91 / 100, 40: 114 / 109;
-// n = 450, 4: 136 / 158, 20: 168 / 177, 80: 205 / 203, 256: 294 / 261; n = 722,
-// 3: 321 / 426, 60: 484 / 544: about even at batch = n^2 / 8000.
+// gain.  Pillar stacks, ms in rounds / in one kernel: n = 162 with 8 matrices
+// 24.2 / 25.5, 32: 26.8 / 25.5; n = 242, 32: 42.5 / 44.6, 64: 45.2 / 46.8, 128:
+// 52.8 / 49.9; n = 338, 40: 70.5 / 76.1, 128: 89.7 / 91.5, 200: 109 / 105; n =
+// 450, 4: 83.5 / 117.5, 80: 127 / 147, 128: 155 / 163, 192: 191 / 190, 256: 225 /
+// 212; n = 722, 3: 163 / 304, 120: 411 / 471, 300: 861 / 883: even near batch =
+// 0.6 (n - 125).
 __host__ constexpr bool qr_split(int n, int batch) {
   const int need = (n - QR_BLOCK) / 10 + 4;
   return n >= 128 && qr_slots(n) >= need && need + QR_MAX_AED <= QR_MAX_OPS &&
-         8000LL * batch <= (long long)n * n;
+         5 * batch <= 3 * (n - 125);
 }
 
 // ---------------------------------------------------------------------------

@@ -31,7 +31,7 @@ def test_rounds_match_numpy(gpu_ctx, n, batch):
         assert np.abs(np.linalg.norm(W[b], axis=0) - 1.0).max() <= 1e-12
 
 
-@pytest.mark.parametrize("n,batch", [(130, 40), (242, 9), (338, 16), (450, 27)])
+@pytest.mark.parametrize("n,batch", [(130, 40), (162, 40), (242, 9), (242, 80), (338, 16), (450, 27)])
 def test_same_matrix_in_any_batch(gpu_ctx, n, batch):
     """A matrix's eigenvalues, their order included, do not depend on the batch it
     is solved in (few matrices iterate in rounds, many in one kernel): a plan that
