@@ -174,6 +174,17 @@ __device__ inline void wave_fence() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
+// A count in LDS by which one wave hands data in LDS to others of its workgroup:
+// what the publishing wave wrote before wave_publish (its other lanes: before a
+// wave_fence in front of it) is there after wave_await(p, v) in any wave, once
+// p has reached v.
+__device__ __forceinline__ void wave_publish(int* p, int v) {
+  __hip_atomic_store(p, v, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+__device__ __forceinline__ void wave_await(const int* p, int v) {
+  while (__hip_atomic_load(p, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP) < v) {}
+}
+
 #define ORCWA_HIP_CHECK(expr)                                                       \
   do {                                                                              \
     hipError_t _e = (expr);                                                         \
