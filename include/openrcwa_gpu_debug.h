@@ -35,6 +35,10 @@ int orcwa_dbg_zgesv(orcwa_gpu_context *ctx, int n, int nrhs, const double *A, co
 int orcwa_dbg_zgeev(orcwa_gpu_context *ctx, int n, const double *A, double *lam, double *W,
                     double *resid, int *info, int batch);
 
+/* The plane rotations of the eigen solver's QR: for each pair (x0, x1) of x,
+ * out = (c, s, r) with c real, c x0 + conj(s) x1 = r and c x1 - s x0 = 0. */
+int orcwa_dbg_rotations(orcwa_gpu_context *ctx, int count, const double *x, double *out);
+
 /* Residual acceptance of the eigen solves of later plans and zgeev calls on
  * this context (default 1e-8, rcwa/MKLEigenSolver.hpp:75-79).  A negative
  * tolerance rejects every solve: it forces the EIG_RESIDUAL status and, in

@@ -145,6 +145,20 @@ int orcwa_dbg_zgeev(orcwa_gpu_context* ctx, int n, const double* A, double* lam,
   return ORCWA_OK;
 }
 
+int orcwa_dbg_rotations(orcwa_gpu_context* ctx, int count, const double* x, double* out) {
+  if (!ctx || count <= 0 || !x || !out) return ORCWA_ERR_ARG;
+  DCHK(hipSetDevice(ctx->device));
+  hipStream_t s = ctx->stream;
+  DBatch in, res;
+  int rc;
+  if ((rc = in.init(s, 2LL * count, 1, x)) || (rc = res.init(s, 3LL * count, 1, nullptr))) return rc;
+  eig_rotations(s, count, in.data, res.data);
+  DCHK(hipGetLastError());
+  DCHK(hipMemcpyAsync(out, res.data, sizeof(cd) * 3 * count, hipMemcpyDeviceToHost, s));
+  DCHK(hipStreamSynchronize(s));
+  return ORCWA_OK;
+}
+
 int orcwa_dbg_set_eig_tolerance(orcwa_gpu_context* ctx, double tol) {
   if (!ctx || tol != tol) return ORCWA_ERR_ARG;
   ctx->eig_tol = tol;
