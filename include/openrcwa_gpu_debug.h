@@ -39,6 +39,10 @@ int orcwa_dbg_zgeev(orcwa_gpu_context *ctx, int n, const double *A, double *lam,
  * out = (c, s, r) with c real, c x0 + conj(s) x1 = r and c x1 - s x0 = 0. */
 int orcwa_dbg_rotations(orcwa_gpu_context *ctx, int count, const double *x, double *out);
 
+/* The shifts of the same QR: of each 2x2 block (column-major) of x, the
+ * eigenvalue nearer to its last entry. */
+int orcwa_dbg_shifts(orcwa_gpu_context *ctx, int count, const double *x, double *out);
+
 /* Residual acceptance of the eigen solves of later plans and zgeev calls on
  * this context (default 1e-8, rcwa/MKLEigenSolver.hpp:75-79).  A negative
  * tolerance rejects every solve: it forces the EIG_RESIDUAL status and, in

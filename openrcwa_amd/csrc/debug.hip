@@ -43,6 +43,24 @@ struct DBatch {
   }
 };
 
+// run(stream, count, in, out) on host arrays of `nin` and `nout` complex an item
+int small_items(orcwa_gpu_context* ctx, int count, int nin, const double* x, int nout, double* out,
+                void (*run)(hipStream_t, int, const cd*, cd*)) {
+  if (!ctx || count <= 0 || !x || !out) return ORCWA_ERR_ARG;
+  DCHK(hipSetDevice(ctx->device));
+  hipStream_t s = ctx->stream;
+  DBatch in, res;
+  int rc;
+  if ((rc = in.init(s, (long long)nin * count, 1, x)) ||
+      (rc = res.init(s, (long long)nout * count, 1, nullptr)))
+    return rc;
+  run(s, count, in.data, res.data);
+  DCHK(hipGetLastError());
+  DCHK(hipMemcpyAsync(out, res.data, sizeof(cd) * nout * count, hipMemcpyDeviceToHost, s));
+  DCHK(hipStreamSynchronize(s));
+  return ORCWA_OK;
+}
+
 }  // namespace
 
 extern "C" {
@@ -146,17 +164,11 @@ int orcwa_dbg_zgeev(orcwa_gpu_context* ctx, int n, const double* A, double* lam,
 }
 
 int orcwa_dbg_rotations(orcwa_gpu_context* ctx, int count, const double* x, double* out) {
-  if (!ctx || count <= 0 || !x || !out) return ORCWA_ERR_ARG;
-  DCHK(hipSetDevice(ctx->device));
-  hipStream_t s = ctx->stream;
-  DBatch in, res;
-  int rc;
-  if ((rc = in.init(s, 2LL * count, 1, x)) || (rc = res.init(s, 3LL * count, 1, nullptr))) return rc;
-  eig_rotations(s, count, in.data, res.data);
-  DCHK(hipGetLastError());
-  DCHK(hipMemcpyAsync(out, res.data, sizeof(cd) * 3 * count, hipMemcpyDeviceToHost, s));
-  DCHK(hipStreamSynchronize(s));
-  return ORCWA_OK;
+  return small_items(ctx, count, 2, x, 3, out, eig_rotations);
+}
+
+int orcwa_dbg_shifts(orcwa_gpu_context* ctx, int count, const double* x, double* out) {
+  return small_items(ctx, count, 4, x, 1, out, eig_shifts);
 }
 
 int orcwa_dbg_set_eig_tolerance(orcwa_gpu_context* ctx, double tol) {

@@ -571,15 +571,16 @@ __device__ __forceinline__ double rsqrt_n(double v) {
   const double p = v * y, q = fma(v, y, -p);
   return fma(0.5 * y, fma(-q, y, fma(-p, y, 1.0)), y);
 }
-// root and reciprocal to about 44 bits, for shifts
-__device__ __forceinline__ double sqrt_shift(double v) {
+// square root and reciprocal of numbers of order 1 to 1 ulp, by the same means
+// (0 for a root of less than 1e-280)
+__device__ __forceinline__ double sqrt_n(double v) {
   if (!(v > 1e-280)) return 0.0;
-  double y = __builtin_amdgcn_rsq(v);
-  y = fma(y, fma(-0.5 * v * y, y, 0.5), y);
-  return v * y;
+  const double y = rsqrt_n(v), r = v * y;
+  return fma(0.5 * y, fma(-r, r, v), r);
 }
-__device__ __forceinline__ double rcp_shift(double v) {
-  const double y = __builtin_amdgcn_rcp(v);
+__device__ __forceinline__ double rcp_n(double v) {
+  double y = __builtin_amdgcn_rcp(v);
+  y = fma(y, fma(-v, y, 1.0), y);
   return fma(y, fma(-v, y, 1.0), y);
 }
 
@@ -718,6 +719,17 @@ __global__ void k_rotations(int count, const cd* x, cd* out) {
 }
 void eig_rotations(hipStream_t s, int count, const cd* x, cd* out) {
   hipLaunchKernelGGL(k_rotations, dim3((count + 255) / 256), dim3(256), 0, s, count, x, out);
+}
+
+// the QR's shifts of 2x2 blocks (column-major), one workgroup a block, for tests
+__global__ void k_shifts(const cd* x, cd* out) {
+  __shared__ alignas(16) cd B[qr_w48::QLD + 2];
+  if (threadIdx.x < 4) B[(threadIdx.x & 1) + (threadIdx.x >> 1) * qr_w48::QLD] = x[4 * blockIdx.x + threadIdx.x];
+  __syncthreads();
+  if (threadIdx.x == 0) out[blockIdx.x] = qr_w48::wilkinson_lds(B, 1);
+}
+void eig_shifts(hipStream_t s, int count, const cd* x, cd* out) {
+  hipLaunchKernelGGL(k_shifts, dim3(count), dim3(64), 0, s, x, out);
 }
 
 __global__ void k_zero_counts(int* a, int n) {

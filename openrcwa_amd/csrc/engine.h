@@ -92,6 +92,8 @@ void zgeev_batched(hipStream_t s, int n, cd* const* A, const cd* const* Aorig, c
                    double tol = kEigTol, int qr_variant = QR_W48, bool host_wait = true);
 // The QR's plane rotations of `count` pairs (x0, x1): out = c, s, r of each.
 void eig_rotations(hipStream_t s, int count, const cd* x, cd* out);
+// The QR's shifts of `count` 2x2 blocks (column-major).
+void eig_shifts(hipStream_t s, int count, const cd* x, cd* out);
 // A[b] = Aorig[b] + diag(1e-11 (i+1) max|Aorig[b]|): the matrix of the
 // reference's recovery solve after a failed residual test
 // (rcwa/MKLEigenSolver.hpp:81-93).

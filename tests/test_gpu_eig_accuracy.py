@@ -58,3 +58,39 @@ def test_rotations_at_the_ends_of_the_range(gpu_ctx, x0, x1):
     # a few roundings of 1.1e-16
     assert unit[0] <= 2e-15
     assert max(abs(x0), abs(x1)) == 0 or back[0] <= 2e-15
+
+
+def _lapack_shift(a, c, b, d):
+    """The eigenvalue of [[a, b], [c, d]] nearer to d as zlahqr forms it, in double."""
+    l1 = lambda z: np.abs(z.real) + np.abs(z.imag)
+    u, x = np.sqrt(b) * np.sqrt(c), 0.5 * (a - d)
+    s = np.maximum(l1(u), l1(x))
+    y = s * np.sqrt((x / s) ** 2 + (u / s) ** 2)
+    y = np.where(x.real * y.real + x.imag * y.imag < 0, -y, y)
+    return d - u * (u / (x + y))
+
+
+@pytest.mark.parametrize("kind", ["dense", "graded", "near_double"])
+def test_shifts_as_accurate_as_in_double(gpu_ctx, kind):
+    rng = np.random.default_rng(5)
+    m = rng.normal(size=(200000, 4)) + 1j * rng.normal(size=(200000, 4))
+    if kind == "graded":
+        m *= np.exp(rng.uniform(-12, 12, m.shape))
+    if kind == "near_double":      # discriminant nearly zero
+        h = 0.5 * (m[:, 0] - m[:, 3])
+        m[:, 1] = -h * h / m[:, 2] * (1 + 1e-9 * rng.normal(size=len(m)))
+    a, c, b, d = np.asarray(m.T, dtype=np.clongdouble)     # column-major
+    l1 = lambda z: np.abs(z.real) + np.abs(z.imag)
+    scale = np.maximum(l1(a - d) / 2, np.maximum(l1(b), l1(c)))
+
+    def residual(sh):
+        # of the characteristic equation, against its terms and the rounding of sh
+        return (np.abs((a - sh) * (d - sh) - b * c) /
+                (scale ** 2 + np.abs(sh) * (np.abs(a - sh) + np.abs(d - sh)))).astype(float)
+
+    sh = _call(gpu_ctx, "orcwa_dbg_shifts", m, 4, 1)[:, 0]
+    got, ref = residual(sh), residual(_lapack_shift(*m.T))
+    assert np.mean(got ** 2) <= np.mean(ref ** 2)
+    assert got.max() <= 1.2 * ref.max()      # (maxima of 2e5 draws scatter)
+    # the eigenvalue nearer to d
+    assert (np.abs(sh - d) <= np.abs(a - sh) * (1 + 1e-9) + 1e-9 * scale).all()
