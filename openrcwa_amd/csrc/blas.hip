@@ -767,20 +767,6 @@ __device__ __forceinline__ double dpp_row_max(double v) {
   return lane_value(dpp_row_reduce_max(v), 15);
 }
 
-// 1 / z: conj(z) times the Newton-refined reciprocal of |z|^2 (2 ulp; a tenth
-// of the instructions of the division), Smith's division near the ends of the
-// range
-__device__ __forceinline__ cd pivot_inv(cd z) {
-  const double n2 = norm2(z);
-  if (n2 > 1e-280 && n2 < 1e280) {
-    double y = __builtin_amdgcn_rcp(n2);
-    y = fma(y, fma(-n2, y, 1.0), y);
-    y = fma(y, fma(-n2, y, 1.0), y);
-    return mk(z.re * y, -z.im * y);
-  }
-  return cinv(z);
-}
-
 template <int J, int T, int WB>
 __device__ __forceinline__ void getrf_reg_step(GetrfRegState<T, WB>& S, cd (&a)[WB]) {
   if constexpr (J < WB) {
@@ -830,7 +816,7 @@ __device__ __forceinline__ void getrf_reg_step(GetrfRegState<T, WB>& S, cd (&a)[
         S.ipiv[(long long)S.b * S.n + c] = bi;
         if (zero) atomicOr(&S.info[S.info_map ? S.info_map[S.b] : S.b], ORCWA_STATUS_SINGULAR);
       }
-      const cd inv = pivot_inv(pv);
+      const cd inv = cinv(pv);
       // rows c and bi trade positions
       S.pos = S.pos == bi ? c : (S.pos == c ? bi : S.pos);
       if (S.pos > c && S.pos < S.n) {
