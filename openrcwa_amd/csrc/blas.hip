@@ -1072,10 +1072,14 @@ void zgetrf_batched(hipStream_t s, int n, cd* const* A, int* ipiv, int* info,
   const cd* const* Ac = (const cd* const*)A;
   for (int k0 = 0, nb; k0 < n; k0 += nb) {
     const int rows = n - k0;
-    // panels of 513 to 1024 rows are kept in registers 16 columns at a time
-    // where launches, not the trailing update's traffic (twice the passes),
-    // take the time: one n = 798 stack 229 -> 219 ms
-    const bool half = rows > GF_T && rows <= GF_T2 && batch <= 64;
+    // Panels of 513 to 1024 rows are kept in registers, 16 columns at a time:
+    // four LUs and their solves of a cascade, ms so / by k_getf2_panel: n = 578, 1
+    // matrix 18.0 / 19.4, 64: 41.8 / 41.8, 256: 120.6 / 118.8; n = 798, 1: 28.5 /
+    // 33.4, 32: 59.1 / 60.7, 64: 93.8 / 90.2, 256: 300 / 277; n = 1058, 1: 43.2 /
+    // 52.8, 256: 617 / 571.  Many matrices pay for twice the passes over the
+    // trailing part, but there the eigen solves take most of the time; and by the
+    // row count alone, because a matrix has to get the same factors in any batch.
+    const bool half = rows > GF_T && rows <= GF_T2;
     nb = std::min(half ? NB2 : NB, rows);
     if (rows <= GF_T)
       hipLaunchKernelGGL((k_getf2_reg<GF_T, NB>), dim3(batch), dim3(GF_T), 0, s, n, k0, nb, A, ipiv,

@@ -26,3 +26,16 @@ def test_pivot_reciprocals_as_accurate_as_in_double(gpu_ctx, ratio):
     # rms of 40000 draws: scatter below 1 %
     assert np.mean(got ** 2) <= 1.02 ** 2 * np.mean(ref ** 2)
     assert got.max() <= 1.1 * ref.max()
+
+
+@pytest.mark.parametrize("n,batch", [(60, 300), (530, 66), (700, 66), (1040, 66)])
+def test_same_solution_in_any_batch(gpu_ctx, n, batch):
+    """A matrix is factored the same way whatever it is batched with, so a plan
+    that runs in chunks agrees with one that does not."""
+    rng = np.random.default_rng(n)
+    A = rng.normal(size=(batch, n, n)) + 1j * rng.normal(size=(batch, n, n))
+    B = rng.normal(size=(batch, n, 33)) + 1j * rng.normal(size=(batch, n, 33))
+    X, info = zgesv(gpu_ctx, A, B)
+    few, info2 = zgesv(gpu_ctx, A[:2], B[:2])
+    assert not info.any() and not info2.any()
+    assert np.array_equal(X[:2], few)
