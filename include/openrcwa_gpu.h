@@ -205,6 +205,9 @@ int orcwa_graph_destroy(orcwa_graph *graph);
  * has three compiled variants (window / shifts per sweep / workgroups per CU:
  * 0 = 48 / 12 / 2, 1 = 32 / 8 / 3, 2 = 64 / 16 / 1) and the GEMMs three tiles
  * for their main block (0 = 64 x 64, 1 = 32 x 64, 2 = 64 x 32).
+ * Batches of few matrices run the QR in rounds over the whole chip, in one form:
+ * the variant is that of the others, and a plan of few matrices leaves it as it
+ * is.  With variants 1 and 2 a matrix's last digits can so depend on its batch.
  * orcwa_plan_autotune executes the plan with each QR variant, then with each
  * tile under the fastest QR variant, keeps the fastest combination for the
  * plan and for later plans of the same layer-matrix size n on the context, and

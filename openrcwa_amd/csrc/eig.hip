@@ -717,6 +717,8 @@ __global__ void k_rotations(int count, const cd* x, cd* out) {
   out[3 * i + 1] = g.s;
   out[3 * i + 2] = g.r;
 }
+bool eig_in_rounds(int n, int batch) { return n >= 3 && qr_split(n, batch); }
+
 void eig_rotations(hipStream_t s, int count, const cd* x, cd* out) {
   hipLaunchKernelGGL(k_rotations, dim3((count + 255) / 256), dim3(256), 0, s, count, x, out);
 }
@@ -1054,7 +1056,8 @@ void zgeev_batched(hipStream_t s, int n, cd* const* A, const cd* const* Aorig, c
   if (ev) (void)hipEventRecord(ev[0], s);
   // zero everything below the first subdiagonal (the Householder vectors)
   hipLaunchKernelGGL(k_zero_below_subdiag, dim3(64, batch), dim3(256), 0, s, n, A);
-  if (qr_variant == QR_W48 && qr_split(n, batch))
+  // (the variant is that of the one kernel; batches in rounds have one form)
+  if (qr_split(n, batch))
     qr_rounds(s, n, A, ws.Z, ws.X, W, reinterpret_cast<int*>(ws.tau), 4 * n * batch, info, batch,
               host_wait);
   else switch (qr_variant) {

@@ -90,6 +90,9 @@ void zgeev_batched(hipStream_t s, int n, cd* const* A, const cd* const* Aorig, c
                    cd* lam, const EigWorkspace& ws, int* info, double* resid,
                    cd* const* scratch, int batch, hipEvent_t* phase_events,
                    double tol = kEigTol, int qr_variant = QR_W48, bool host_wait = true);
+// Whether a batch's QR runs in rounds over the whole chip, not in the one kernel
+// whose variant qr_variant names.
+bool eig_in_rounds(int n, int batch);
 // The QR's plane rotations of `count` pairs (x0, x1): out = c, s, r of each.
 void eig_rotations(hipStream_t s, int count, const cd* x, cd* out);
 // The QR's shifts of `count` 2x2 blocks (column-major).

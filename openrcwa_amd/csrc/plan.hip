@@ -1889,10 +1889,16 @@ int orcwa_plan_autotune(orcwa_plan* p, int* qr_variant, int* gemm_tile) {
     ms = p->phase_ms[0];
     return ORCWA_OK;
   };
-  // the QR variants with the default tile, then the tiles with the best QR
-  int best_qr = QR_W48, best_tile = GEMM_TILE_64x64;
+  // The QR variants with the default tile, then the tiles with the best QR.  A
+  // plan whose eigen solves all run in rounds says nothing about the variants:
+  // the one in use for this n stays.
+  bool one_kernel = false;
+  for (const ChunkTables& ct : p->chunks)
+    one_kernel = one_kernel || (ct.nprob > 0 && !eig_in_rounds(p->n, ct.nprob));
+  const int first = one_kernel ? 0 : p->qr_variant, last = one_kernel ? QR_NVARIANTS - 1 : first;
+  int best_qr = first, best_tile = GEMM_TILE_64x64;
   double best = 1e300, ms = 0.0;
-  for (int q = 0; q < QR_NVARIANTS; ++q) {
+  for (int q = first; q <= last; ++q) {
     const int rc = timed(q, GEMM_TILE_64x64, ms);
     if (rc != ORCWA_OK) return rc;
     if (ms > 0.0 && ms < best) {
