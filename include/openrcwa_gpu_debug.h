@@ -29,11 +29,23 @@ int orcwa_dbg_zgemm(orcwa_gpu_context *ctx, int M, int N, int K, const double *a
 int orcwa_dbg_zgesv(orcwa_gpu_context *ctx, int n, int nrhs, const double *A, const double *B,
                     double *X, int *info, int batch);
 
+/* A = P L U in place for a batch of n x n matrices: ipiv[b][k] (from 0) is the
+ * row that traded places with row k, the lowest of those with the largest
+ * |re| + |im|; info as for zgesv. */
+int orcwa_dbg_zgetrf(orcwa_gpu_context *ctx, int n, double *A, int *ipiv, int *info, int batch);
+
 /* Eigenvalues lam[b][n] and unit-norm right eigenvectors W[b] (n x n) of a
  * batch of general complex matrices; resid[b] = ||AW - W diag(lam)||max/||A||max;
  * info[b] status bits. */
 int orcwa_dbg_zgeev(orcwa_gpu_context *ctx, int n, const double *A, double *lam, double *W,
                     double *resid, int *info, int batch);
+
+/* The same with the QR's route given: rounds < 0 as the batch wants it, 0 in one
+ * kernel, k > 0 in k rounds over the whole chip and then in one kernel from
+ * where these left off (ORCWA_ERR_ARG where n is too small for rounds);
+ * maxsweep > 0: sweeps after which a matrix is given up (ORCWA_STATUS_NOCONV). */
+int orcwa_dbg_zgeev_route(orcwa_gpu_context *ctx, int n, const double *A, double *lam, double *W,
+                          double *resid, int *info, int batch, int rounds, int maxsweep);
 
 /* The plane rotations of the eigen solver's QR: for each pair (x0, x1) of x,
  * out = (c, s, r) with c real, c x0 + conj(s) x1 = r and c x1 - s x0 = 0. */

@@ -122,9 +122,40 @@ int orcwa_dbg_zgesv(orcwa_gpu_context* ctx, int n, int nrhs, const double* A, co
   return ORCWA_OK;
 }
 
+int orcwa_dbg_zgetrf(orcwa_gpu_context* ctx, int n, double* A, int* ipiv, int* info, int batch) {
+  if (!ctx || n <= 0 || batch <= 0) return ORCWA_ERR_ARG;
+  DCHK(hipSetDevice(ctx->device));
+  orcwa::ctx_trim(ctx);   // cached plan buffers go back to the device
+  hipStream_t s = ctx->stream;
+  DBatch a;
+  int rc;
+  if ((rc = a.init(s, (long long)n * n, batch, A))) return rc;
+  int *dpiv = nullptr, *dinfo = nullptr;
+  DCHK(hipMalloc(&dpiv, sizeof(int) * n * batch));
+  DCHK(hipMalloc(&dinfo, sizeof(int) * batch));
+  DCHK(hipMemsetAsync(dinfo, 0, sizeof(int) * batch, s));
+  zgetrf_batched(s, n, a.table, dpiv, dinfo, nullptr, batch);
+  hipError_t e = hipGetLastError();
+  if (e == hipSuccess)
+    e = hipMemcpyAsync(A, a.data, sizeof(cd) * n * n * batch, hipMemcpyDeviceToHost, s);
+  if (e == hipSuccess) e = hipMemcpyAsync(ipiv, dpiv, sizeof(int) * n * batch, hipMemcpyDeviceToHost, s);
+  if (e == hipSuccess) e = hipMemcpyAsync(info, dinfo, sizeof(int) * batch, hipMemcpyDeviceToHost, s);
+  if (e == hipSuccess) e = hipStreamSynchronize(s);
+  (void)hipFree(dpiv);
+  (void)hipFree(dinfo);
+  DCHK(e);
+  return ORCWA_OK;
+}
+
 int orcwa_dbg_zgeev(orcwa_gpu_context* ctx, int n, const double* A, double* lam, double* W,
                     double* resid, int* info, int batch) {
+  return orcwa_dbg_zgeev_route(ctx, n, A, lam, W, resid, info, batch, -1, 0);
+}
+
+int orcwa_dbg_zgeev_route(orcwa_gpu_context* ctx, int n, const double* A, double* lam, double* W,
+                          double* resid, int* info, int batch, int rounds, int maxsweep) {
   if (!ctx || n <= 0 || batch <= 0) return ORCWA_ERR_ARG;
+  if (rounds > 0 && !eig_rounds_fit(n)) return ORCWA_ERR_ARG;
   DCHK(hipSetDevice(ctx->device));
   orcwa::ctx_trim(ctx);   // cached plan buffers go back to the device
   hipStream_t s = ctx->stream;
@@ -148,7 +179,7 @@ int orcwa_dbg_zgeev(orcwa_gpu_context* ctx, int n, const double* A, double* lam,
   ws.X = x.table;
   ws.tau = dtau;
   zgeev_batched(s, n, a.table, (const cd* const*)ao.table, w.table, dlam, ws, dinfo, dres,
-                x.table, batch, nullptr, ctx->eig_tol);
+                x.table, batch, nullptr, ctx->eig_tol, QR_W48, true, QrRoute{rounds, maxsweep});
   hipError_t e = hipGetLastError();
   if (e == hipSuccess) e = hipMemcpyAsync(lam, dlam, sizeof(cd) * n * batch, hipMemcpyDeviceToHost, s);
   if (e == hipSuccess) e = hipMemcpyAsync(W, w.data, sizeof(cd) * nn * batch, hipMemcpyDeviceToHost, s);

@@ -664,10 +664,12 @@ __host__ __device__ constexpr int qr_slots(int n) {
 // 450, 4: 83.5 / 117.5, 80: 127 / 147, 128: 155 / 163, 192: 191 / 190, 256: 225 /
 // 212; n = 722, 3: 163 / 304, 120: 411 / 471, 300: 861 / 883: even near batch =
 // 0.6 (n - 125).
-__host__ constexpr bool qr_split(int n, int batch) {
+__host__ constexpr bool qr_fits(int n) {
   const int need = (n - QR_BLOCK) / 10 + 4;
-  return n >= 128 && qr_slots(n) >= need && need + QR_MAX_AED <= QR_MAX_OPS &&
-         5 * batch <= 3 * (n - 125);
+  return n >= 128 && qr_slots(n) >= need && need + QR_MAX_AED <= QR_MAX_OPS;
+}
+__host__ constexpr bool qr_split(int n, int batch) {
+  return qr_fits(n) && 5 * batch <= 3 * (n - 125);
 }
 
 // ---------------------------------------------------------------------------
@@ -717,7 +719,8 @@ __global__ void k_rotations(int count, const cd* x, cd* out) {
   out[3 * i + 1] = g.s;
   out[3 * i + 2] = g.r;
 }
-bool eig_in_rounds(int n, int batch) { return n >= 3 && qr_split(n, batch); }
+bool eig_in_rounds(int n, int batch) { return qr_split(n, batch); }
+bool eig_rounds_fit(int n) { return qr_fits(n); }
 
 void eig_rotations(hipStream_t s, int count, const cd* x, cd* out) {
   hipLaunchKernelGGL(k_rotations, dim3((count + 255) / 256), dim3(256), 0, s, count, x, out);
@@ -745,13 +748,13 @@ __host__ constexpr int qr_fixed_rounds(int n) { return 8 + n / 6; }
 // left from a counter per round, read back only when about as many sweeps have
 // run as an RCWA matrix takes (n / 12), then every few rounds: a round that
 // finds nothing to do costs two empty launches.  Where the host may not wait (a
-// graph is captured) the rounds are qr_fixed_rounds(n), and the kernel of one workgroup
-// a matrix takes on whatever is left: the same iteration, so a replay agrees with
+// graph is captured) there are `fixed` rounds, and the kernel of one workgroup a
+// matrix takes on whatever is left: the same iteration, so a replay agrees with
 // the eager solve.
 static void qr_rounds(hipStream_t s, int n, cd* const* A, cd* const* Z, cd* const* X,
                       cd* const* W, int* counts, int ncounts, int* info, int batch,
-                      bool host_wait) {
-  const int maxsweep = 40 + 3 * n, strips = 3 * ((n + 63) / 64);
+                      bool host_wait, int fixed, int maxsweep) {
+  const int strips = 3 * ((n + 63) / 64);
   const int nc = std::min(ncounts, 1024);
   int round = 0, check = std::max(2, n / 13);
   while (true) {
@@ -761,7 +764,7 @@ static void qr_rounds(hipStream_t s, int n, cd* const* A, cd* const* Z, cd* cons
                        X, W, info, counts, maxsweep);
     hipLaunchKernelGGL(qr_w48::k_qr_apply, dim3(strips * batch), dim3(256), 0, s, n, batch, A, Z, X, W);
     ++round;
-    if (!host_wait && round == qr_fixed_rounds(n)) {
+    if (!host_wait && round >= fixed) {
       hipLaunchKernelGGL(qr_w48::k_qr_ms, dim3(batch), dim3(256), 0, s, n, A, Z,
                          (const cd* const*)X, info, maxsweep);
       return;
@@ -1012,7 +1015,7 @@ void eig_recover_scatter(hipStream_t s, int n, int m, const int* idx, const cd* 
 void zgeev_batched(hipStream_t s, int n, cd* const* A, const cd* const* Aorig, cd* const* W,
                    cd* lam, const EigWorkspace& ws, int* info, double* resid,
                    cd* const* scratch, int batch, hipEvent_t* ev, double tol, int qr_variant,
-                   bool host_wait) {
+                   bool host_wait, const QrRoute& route) {
   if (batch <= 0 || n <= 0) return;
   const cd* const* Ac = (const cd* const*)A;
   if (n >= 3) {
@@ -1057,21 +1060,23 @@ void zgeev_batched(hipStream_t s, int n, cd* const* A, const cd* const* Aorig, c
   // zero everything below the first subdiagonal (the Householder vectors)
   hipLaunchKernelGGL(k_zero_below_subdiag, dim3(64, batch), dim3(256), 0, s, n, A);
   // (the variant is that of the one kernel; batches in rounds have one form)
-  if (qr_split(n, batch))
+  const int maxsweep = route.maxsweep > 0 ? route.maxsweep : 40 + 3 * n;
+  if (route.rounds < 0 ? qr_split(n, batch) : route.rounds > 0)
     qr_rounds(s, n, A, ws.Z, ws.X, W, reinterpret_cast<int*>(ws.tau), 4 * n * batch, info, batch,
-              host_wait);
+              host_wait && route.rounds < 0, route.rounds > 0 ? route.rounds : qr_fixed_rounds(n),
+              maxsweep);
   else switch (qr_variant) {
     case QR_W32:
       hipLaunchKernelGGL(qr_w32::k_qr_ms, dim3(batch), dim3(256), 0, s, n, A, ws.Z, nullptr,
-                         info, 40 + 3 * n);
+                         info, maxsweep);
       break;
     case QR_W64:
       hipLaunchKernelGGL(qr_w64::k_qr_ms, dim3(batch), dim3(256), 0, s, n, A, ws.Z, nullptr,
-                         info, 40 + 3 * n);
+                         info, maxsweep);
       break;
     default:
       hipLaunchKernelGGL(qr_w48::k_qr_ms, dim3(batch), dim3(256), 0, s, n, A, ws.Z, nullptr,
-                         info, 40 + 3 * n);
+                         info, maxsweep);
   }
   if (ev) (void)hipEventRecord(ev[1], s);
   if (n >= 64)

@@ -86,13 +86,21 @@ struct EigWorkspace {
 // Variants of the multishift QR (window / shifts / workgroups per CU):
 // QR_W48 48 / 12 / 2 (default), QR_W32 32 / 8 / 3, QR_W64 64 / 16 / 1.
 enum QrVariant { QR_W48 = 0, QR_W32 = 1, QR_W64 = 2, QR_NVARIANTS = 3 };
+// How the QR runs, for tests of its routes (by default as the batch wants it).
+struct QrRoute {
+  int rounds = -1;    // 0: in one kernel; k > 0: k rounds, then the one kernel on what is left
+  int maxsweep = 0;   // > 0: sweeps after which a matrix is given up
+};
 void zgeev_batched(hipStream_t s, int n, cd* const* A, const cd* const* Aorig, cd* const* W,
                    cd* lam, const EigWorkspace& ws, int* info, double* resid,
                    cd* const* scratch, int batch, hipEvent_t* phase_events,
-                   double tol = kEigTol, int qr_variant = QR_W48, bool host_wait = true);
+                   double tol = kEigTol, int qr_variant = QR_W48, bool host_wait = true,
+                   const QrRoute& route = QrRoute());
 // Whether a batch's QR runs in rounds over the whole chip, not in the one kernel
 // whose variant qr_variant names.
 bool eig_in_rounds(int n, int batch);
+// Whether rounds are possible at this n.
+bool eig_rounds_fit(int n);
 // The QR's plane rotations of `count` pairs (x0, x1): out = c, s, r of each.
 void eig_rotations(hipStream_t s, int count, const cd* x, cd* out);
 // The QR's shifts of `count` 2x2 blocks (column-major).

@@ -1,8 +1,11 @@
 """The LU's pivots: the accuracy of their reciprocals against double precision."""
+import ctypes
+
 import numpy as np
 import pytest
 
-from .gpu_helpers import zgesv
+from openrcwa_amd import _lib
+from .gpu_helpers import fortran_batch, from_fortran, zgesv
 
 pytestmark = pytest.mark.gpu
 
@@ -39,3 +42,76 @@ def test_same_solution_in_any_batch(gpu_ctx, n, batch):
     few, info2 = zgesv(gpu_ctx, A[:2], B[:2])
     assert not info.any() and not info2.any()
     assert np.array_equal(X[:2], few)
+
+
+def zgetrf(ctx, A):
+    fn = _lib.load().orcwa_dbg_zgetrf
+    q = ctypes.POINTER(ctypes.c_int)
+    fn.argtypes = [ctypes.c_void_p, ctypes.c_int, ctypes.POINTER(ctypes.c_double), q, q,
+                   ctypes.c_int]
+    batch, n, _ = A.shape
+    a = fortran_batch(A)
+    ipiv, info = np.zeros((batch, n), dtype=np.int32), np.zeros(batch, dtype=np.int32)
+    _lib.check(fn(ctx.handle, n, a.ctypes.data_as(ctypes.POINTER(ctypes.c_double)),
+                  ipiv.ctypes.data_as(q), info.ctypes.data_as(q), batch), "orcwa_dbg_zgetrf")
+    return from_fortran(a, n, n), ipiv, info
+
+
+def eliminate(a):
+    """LU with the lowest row of the largest |re| + |im| as the pivot; also the
+    number of columns where more than one row has it."""
+    a, n, ties = a.copy(), len(a), 0
+    piv = np.zeros(n, dtype=np.int32)
+    for k in range(n):
+        m = np.abs(a[k:, k].real) + np.abs(a[k:, k].imag)
+        ties += (m == m.max()).sum() > 1
+        piv[k] = k + int(np.argmax(m))
+        a[[k, piv[k]]] = a[[piv[k], k]]
+        a[k + 1:, k] /= a[k, k]
+        a[k + 1:, k + 1:] -= np.outer(a[k + 1:, k], a[k, k + 1:])
+    return a, piv, ties
+
+
+# one wave; all 512 rows; more rows than that in the first panels, 1024; more again
+@pytest.mark.parametrize("blocks", [(64,), (32, 8), (512,), (512, 32, 32), (512, 256), (1024,),
+                                    (1024, 64)])
+def test_ties_take_the_lowest_row(gpu_ctx, blocks):
+    """Hadamard blocks, their rows shuffled and turned by units: nearly every column
+    has ties for its pivot, within a wave and across waves, and elimination is
+    exact (every entry is a small multiple of a power of two)."""
+    n = sum(blocks)
+    rng = np.random.default_rng(n)
+    mats = []
+    for _ in range(2):
+        a = np.zeros((n, n), dtype=complex)
+        r = 0
+        for m in blocks:
+            h = np.ones((1, 1))
+            while len(h) < m:
+                h = np.block([[h, h], [h, -h]])
+            a[r:r + m, r:r + m] = h
+            r += m
+        mats.append(np.array([1, 1j, -1, -1j])[rng.integers(0, 4, n), None] * a[rng.permutation(n)])
+    lu, ipiv, info = zgetrf(gpu_ctx, np.array(mats))
+    assert not info.any()
+    for b in range(2):
+        ref, piv, ties = eliminate(mats[b])
+        assert ties > n // 4
+        assert np.array_equal(ipiv[b], piv)
+        assert np.array_equal(lu[b], ref)
+
+
+@pytest.mark.parametrize("n", [40, 300, 600, 1030])
+def test_a_matrix_that_is_not_finite(gpu_ctx, n):
+    """It ends, its pivots are rows of the matrix, and the others of its batch are
+    as without it."""
+    rng = np.random.default_rng(n)
+    a = rng.normal(size=(4, n, n)) + 1j * rng.normal(size=(4, n, n))
+    ref = zgetrf(gpu_ctx, a)
+    a[1][:, n // 2] = np.nan
+    a[2][n // 3, n // 4] = np.inf
+    lu, ipiv, info = zgetrf(gpu_ctx, a)
+    assert ((ipiv >= np.arange(n)) & (ipiv < n)).all()
+    for b in (0, 3):
+        assert np.array_equal(lu[b], ref[0][b]) and np.array_equal(ipiv[b], ref[1][b])
+        assert info[b] == 0
