@@ -983,10 +983,15 @@ __global__ __launch_bounds__(256) void k_apply_perm(int n, int nrhs, int ncw, co
 // column (a column's 32-row segment is 512 contiguous bytes; read directly,
 // the lanes of a wave would each touch another column).  All slabs are loaded
 // before the first is staged: one memory latency instead of four.
-constexpr int TR_SLAB = 8;
-template <bool UNIT_LOWER, int TPB>
-__global__ __launch_bounds__(TPB) void k_trsm_block(int n, int k0, int nb, int c0, int ncols,
-                                                    const cd* const* Lp, cd* const* Xp) {
+// 256 columns a workgroup, also where few workgroups result: 64 took as long or
+// longer from 1 to 1024 matrices (four LUs and solves of a cascade, ms by 256 / 64:
+// n = 98, 1 matrix 2.14 / 2.16, 128: 2.50 / 2.61; n = 450, 1: 13.1 / 13.2, 256:
+// 62.7 / 65.0; n = 722, 1: 23.7 / 24.0, 1024: 851 / 863).
+constexpr int TR_SLAB = 8, TR_COLS = 256;
+template <bool UNIT_LOWER>
+__global__ __launch_bounds__(TR_COLS) void k_trsm_block(int n, int k0, int nb, int c0, int ncols,
+                                                        const cd* const* Lp, cd* const* Xp) {
+  constexpr int TPB = TR_COLS;
   __shared__ alignas(16) cd sT[NB][NB];
   __shared__ alignas(16) cd sX[TPB][TR_SLAB + 1];
   const int b = blockIdx.y;
@@ -1053,17 +1058,11 @@ __global__ __launch_bounds__(TPB) void k_trsm_block(int n, int k0, int nb, int c
   }
 }
 
-// 256 columns a workgroup where that fills the chip, else 64 (one wave: more
-// workgroups, no waiting between waves)
 template <bool UNIT_LOWER>
 static void trsm_block(hipStream_t s, int n, int k0, int nb, int c0, int ncols,
                        const cd* const* L, cd* const* X, int batch) {
-  if ((long long)((ncols + 255) / 256) * batch >= 512)
-    hipLaunchKernelGGL((k_trsm_block<UNIT_LOWER, 256>), dim3((ncols + 255) / 256, batch), dim3(256),
-                       0, s, n, k0, nb, c0, ncols, L, X);
-  else
-    hipLaunchKernelGGL((k_trsm_block<UNIT_LOWER, 64>), dim3((ncols + 63) / 64, batch), dim3(64), 0,
-                       s, n, k0, nb, c0, ncols, L, X);
+  hipLaunchKernelGGL((k_trsm_block<UNIT_LOWER>), dim3((ncols + TR_COLS - 1) / TR_COLS, batch),
+                     dim3(TR_COLS), 0, s, n, k0, nb, c0, ncols, L, X);
 }
 
 void zgetrf_batched(hipStream_t s, int n, cd* const* A, int* ipiv, int* info,
