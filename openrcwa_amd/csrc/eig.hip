@@ -11,7 +11,9 @@
 //   4. eigenvectors of the triangular T by back substitution (with the
 //      smin = max(ulp |t_jj|, smlnum) pivot guard), W = Z X, unit 2-norm columns
 //   5. the reference's acceptance test ||A W - W diag(l)||max / ||A||max <= 1e-8
-// One workgroup owns one matrix; matrices live in HBM (column-major).
+// Matrices live in HBM (column-major).  The serial parts run on one workgroup a
+// matrix; what reads or writes whole matrices (the Hessenberg matvec, the block
+// updates, for few matrices the QR's updates) on the whole chip.
 #include <algorithm>
 #include <cfloat>
 
@@ -357,7 +359,7 @@ static void hess_panel(hipStream_t s, int n, int i0, int nb, cd* const* A, cd* t
   const int strips = (n - i0 - 1 + 63) / 64;
   // column ranges of a width that depends on n alone, so that a matrix's sums,
   // and with them its eigenvalues' order, do not depend on what it is batched
-  // with; at least 32 columns, at most HB ranges
+  // with; at least 64 columns, at most HB ranges
   const int cw = std::max(64, (n + HB - 1) / HB), nch = (n - i0 - 2 + cw) / cw;
   for (int j = 0; j <= nb; ++j) {
     hipLaunchKernelGGL(k_hess_col, dim3(batch), dim3(HC_T), n * sizeof(cd), s, n, i0, j, nb, nch,
@@ -663,7 +665,9 @@ __host__ __device__ constexpr int qr_slots(int n) {
 // 52.8 / 49.9; n = 338, 40: 70.5 / 76.1, 128: 89.7 / 91.5, 200: 109 / 105; n =
 // 450, 4: 83.5 / 117.5, 80: 127 / 147, 128: 155 / 163, 192: 191 / 190, 256: 225 /
 // 212; n = 722, 3: 163 / 304, 120: 411 / 471, 300: 861 / 883: even near batch =
-// 0.6 (n - 125).
+// 0.6 (n - 125).  Further out, the eigen solve alone: n = 1058, 4: 273 / 687, 256:
+// 1344 / 1412, 560: 3024 / 3169; n = 1250, 4: 386 / 1071, 280: 2570 / 2850; n =
+// 1922, 4: 1060 / 3513, 64: 2561 / 4546, 384: 10962 / 11291.
 __host__ constexpr bool qr_fits(int n) {
   const int need = (n - QR_BLOCK) / 10 + 4;
   return n >= 128 && qr_slots(n) >= need && need + QR_MAX_AED <= QR_MAX_OPS;
@@ -741,13 +745,14 @@ __global__ void k_zero_counts(int* a, int n) {
   for (int i = threadIdx.x; i < n; i += blockDim.x) a[i] = 0;
 }
 
-// about twice what an RCWA matrix takes
+// rounds where the host cannot see how many are needed: about 1.6 times what an
+// RCWA matrix takes (53 at n = 450, 89 at n = 798)
 __host__ constexpr int qr_fixed_rounds(int n) { return 8 + n / 6; }
 
 // The rounds of the two-kernel form.  The host learns how many matrices are
-// left from a counter per round, read back only when about as many sweeps have
-// run as an RCWA matrix takes (n / 12), then every few rounds: a round that
-// finds nothing to do costs two empty launches.  Where the host may not wait (a
+// left from a counter per round, read back from round n / 13 on (an RCWA matrix
+// takes about n / 9 sweeps), then after every second round: a round that finds
+// nothing to do costs two empty launches.  Where the host may not wait (a
 // graph is captured) there are `fixed` rounds, and the kernel of one workgroup a
 // matrix takes on whatever is left: the same iteration, so a replay agrees with
 // the eager solve.
