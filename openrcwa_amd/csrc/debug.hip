@@ -178,9 +178,10 @@ int orcwa_dbg_zgeev_route(orcwa_gpu_context* ctx, int n, const double* A, double
   ws.Z = z.table;
   ws.X = x.table;
   ws.tau = dtau;
-  zgeev_batched(s, n, a.table, (const cd* const*)ao.table, w.table, dlam, ws, dinfo, dres,
-                x.table, batch, nullptr, ctx->eig_tol, QR_W48, true, QrRoute{rounds, maxsweep});
-  hipError_t e = hipGetLastError();
+  hipError_t e = zgeev_batched(s, n, a.table, (const cd* const*)ao.table, w.table, dlam, ws, dinfo,
+                               dres, x.table, batch, nullptr, ctx->eig_tol, QR_W48, true,
+                               QrRoute{rounds, maxsweep});
+  if (e == hipSuccess) e = hipGetLastError();
   if (e == hipSuccess) e = hipMemcpyAsync(lam, dlam, sizeof(cd) * n * batch, hipMemcpyDeviceToHost, s);
   if (e == hipSuccess) e = hipMemcpyAsync(W, w.data, sizeof(cd) * nn * batch, hipMemcpyDeviceToHost, s);
   if (e == hipSuccess) e = hipMemcpyAsync(resid, dres, sizeof(double) * batch, hipMemcpyDeviceToHost, s);

@@ -756,9 +756,9 @@ __host__ constexpr int qr_fixed_rounds(int n) { return 8 + n / 6; }
 // graph is captured) there are `fixed` rounds, and the kernel of one workgroup a
 // matrix takes on whatever is left: the same iteration, so a replay agrees with
 // the eager solve.
-static void qr_rounds(hipStream_t s, int n, cd* const* A, cd* const* Z, cd* const* X,
-                      cd* const* W, int* counts, int ncounts, int* info, int batch,
-                      bool host_wait, int fixed, int maxsweep) {
+static hipError_t qr_rounds(hipStream_t s, int n, cd* const* A, cd* const* Z, cd* const* X,
+                            cd* const* W, int* counts, int ncounts, int* info, int batch,
+                            bool host_wait, int fixed, int maxsweep) {
   const int strips = 3 * ((n + 63) / 64);
   const int nc = std::min(ncounts, 1024);
   int round = 0, check = std::max(2, n / 13);
@@ -772,14 +772,14 @@ static void qr_rounds(hipStream_t s, int n, cd* const* A, cd* const* Z, cd* cons
     if (!host_wait && round >= fixed) {
       hipLaunchKernelGGL(qr_w48::k_qr_ms, dim3(batch), dim3(256), 0, s, n, A, Z,
                          (const cd* const*)X, info, maxsweep);
-      return;
+      return hipSuccess;
     }
     if (!host_wait || round < check) continue;
     check = round + 2;
     int left = 0;
-    if (hipMemcpyAsync(&left, counts + slot, sizeof(int), hipMemcpyDeviceToHost, s) != hipSuccess ||
-        hipStreamSynchronize(s) != hipSuccess || left == 0)
-      return;
+    hipError_t e = hipMemcpyAsync(&left, counts + slot, sizeof(int), hipMemcpyDeviceToHost, s);
+    if (e == hipSuccess) e = hipStreamSynchronize(s);
+    if (e != hipSuccess || left == 0) return e;
   }
 }
 
@@ -1017,11 +1017,11 @@ void eig_recover_scatter(hipStream_t s, int n, int m, const int* idx, const cd* 
                      res_k, lam, info, resid);
 }
 
-void zgeev_batched(hipStream_t s, int n, cd* const* A, const cd* const* Aorig, cd* const* W,
-                   cd* lam, const EigWorkspace& ws, int* info, double* resid,
-                   cd* const* scratch, int batch, hipEvent_t* ev, double tol, int qr_variant,
-                   bool host_wait, const QrRoute& route) {
-  if (batch <= 0 || n <= 0) return;
+hipError_t zgeev_batched(hipStream_t s, int n, cd* const* A, const cd* const* Aorig, cd* const* W,
+                         cd* lam, const EigWorkspace& ws, int* info, double* resid,
+                         cd* const* scratch, int batch, hipEvent_t* ev, double tol, int qr_variant,
+                         bool host_wait, const QrRoute& route) {
+  if (batch <= 0 || n <= 0) return hipSuccess;
   const cd* const* Ac = (const cd* const*)A;
   if (n >= 3) {
     if (n >= 128)
@@ -1066,11 +1066,13 @@ void zgeev_batched(hipStream_t s, int n, cd* const* A, const cd* const* Aorig, c
   hipLaunchKernelGGL(k_zero_below_subdiag, dim3(64, batch), dim3(256), 0, s, n, A);
   // (the variant is that of the one kernel; batches in rounds have one form)
   const int maxsweep = route.maxsweep > 0 ? route.maxsweep : 40 + 3 * n;
-  if (route.rounds < 0 ? qr_split(n, batch) : route.rounds > 0)
-    qr_rounds(s, n, A, ws.Z, ws.X, W, reinterpret_cast<int*>(ws.tau), 4 * n * batch, info, batch,
-              host_wait && route.rounds < 0, route.rounds > 0 ? route.rounds : qr_fixed_rounds(n),
-              maxsweep);
-  else switch (qr_variant) {
+  if (route.rounds < 0 ? qr_split(n, batch) : route.rounds > 0) {
+    const hipError_t e =
+        qr_rounds(s, n, A, ws.Z, ws.X, W, reinterpret_cast<int*>(ws.tau), 4 * n * batch, info,
+                  batch, host_wait && route.rounds < 0,
+                  route.rounds > 0 ? route.rounds : qr_fixed_rounds(n), maxsweep);
+    if (e != hipSuccess) return e;
+  } else switch (qr_variant) {
     case QR_W32:
       hipLaunchKernelGGL(qr_w32::k_qr_ms, dim3(batch), dim3(256), 0, s, n, A, ws.Z, nullptr,
                          info, maxsweep);
@@ -1105,6 +1107,7 @@ void zgeev_batched(hipStream_t s, int n, cd* const* A, const cd* const* Aorig, c
                        resid, info, tol, batch);
   }
   if (ev) (void)hipEventRecord(ev[2], s);
+  return hipSuccess;
 }
 
 }  // namespace orcwa

@@ -77,7 +77,8 @@ void copy_batched(hipStream_t s, long long count, const cd* const* A, cd* const*
 // ORCWA_STATUS_EIG_RESIDUAL); status bits are or-ed into info[b].  resid[b]
 // receives the relative residual.  host_wait: the launcher may wait for the
 // stream (to see how many rounds of the QR are still needed); in a stream
-// capture it may not.
+// capture it may not.  Returns the error of such a wait: the rest is then not
+// launched, and the results are not there.
 struct EigWorkspace {
   cd** Z;        // [batch] n*n
   cd** X;        // [batch] n*n
@@ -91,11 +92,11 @@ struct QrRoute {
   int rounds = -1;    // 0: in one kernel; k > 0: k rounds, then the one kernel on what is left
   int maxsweep = 0;   // > 0: sweeps after which a matrix is given up
 };
-void zgeev_batched(hipStream_t s, int n, cd* const* A, const cd* const* Aorig, cd* const* W,
-                   cd* lam, const EigWorkspace& ws, int* info, double* resid,
-                   cd* const* scratch, int batch, hipEvent_t* phase_events,
-                   double tol = kEigTol, int qr_variant = QR_W48, bool host_wait = true,
-                   const QrRoute& route = QrRoute());
+hipError_t zgeev_batched(hipStream_t s, int n, cd* const* A, const cd* const* Aorig, cd* const* W,
+                         cd* lam, const EigWorkspace& ws, int* info, double* resid,
+                         cd* const* scratch, int batch, hipEvent_t* phase_events,
+                         double tol = kEigTol, int qr_variant = QR_W48, bool host_wait = true,
+                         const QrRoute& route = QrRoute());
 // Whether a batch's QR runs in rounds over the whole chip, not in the one kernel
 // whose variant qr_variant names.
 bool eig_in_rounds(int n, int batch);

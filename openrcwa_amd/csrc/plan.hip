@@ -1098,11 +1098,13 @@ static int eig_recover(orcwa_plan* p, const ChunkTables& ct, hipStream_t s,
     int* info_k = reinterpret_cast<int*>(buf + o_info);
     double* res_k = reinterpret_cast<double*>(buf + o_res);
     eig_perturb_batched(s, n, tAo, tA, m);
-    zgeev_batched(s, n, tA, tAo, tW, lam_k, ws, info_k, res_k, ws.X, m, nullptr,
-                  p->ctx->eig_tol, p->qr_variant);
-    eig_recover_scatter(s, n, m, reinterpret_cast<const int*>(buf + o_idx), lam_k, info_k,
-                        res_k, p->d_lam, p->d_pinfo + ct.prob_base, p->d_resid + ct.prob_base);
-    e = hipGetLastError();
+    e = zgeev_batched(s, n, tA, tAo, tW, lam_k, ws, info_k, res_k, ws.X, m, nullptr,
+                      p->ctx->eig_tol, p->qr_variant);
+    if (e == hipSuccess) {
+      eig_recover_scatter(s, n, m, reinterpret_cast<const int*>(buf + o_idx), lam_k, info_k,
+                          res_k, p->d_lam, p->d_pinfo + ct.prob_base, p->d_resid + ct.prob_base);
+      e = hipGetLastError();
+    }
   }
   if (e == hipSuccess) e = hipStreamSynchronize(s);
   (void)hipFree(buf);
@@ -1271,10 +1273,10 @@ static int plan_run(orcwa_plan* p, hipStream_t s, bool graph) {
       ws.X = p->dev<cd**>(ct.pX);
       ws.tau = p->d_tau;
       HIPCHK(record(5));
-      zgeev_batched(s, n, A, p->dev<const cd* const*>(ct.pAorig), Wp, p->d_lam, ws,
-                    p->d_pinfo + ct.prob_base, p->d_resid + ct.prob_base,
-                    p->dev<cd* const*>(ct.pX), np, nullptr, p->ctx->eig_tol, p->qr_variant,
-                    !graph);
+      HIPCHK(zgeev_batched(s, n, A, p->dev<const cd* const*>(ct.pAorig), Wp, p->d_lam, ws,
+                           p->d_pinfo + ct.prob_base, p->d_resid + ct.prob_base,
+                           p->dev<cd* const*>(ct.pX), np, nullptr, p->ctx->eig_tol, p->qr_variant,
+                           !graph));
       if (!graph) {
         const int rc = eig_recover(p, ct, s, recovered);
         if (rc != ORCWA_OK) return rc;
